@@ -106,9 +106,12 @@ long long sht_plan_device_bytes(const sht_plan *plan);
  *                     whose product shares the vector's P slices (1, for
  *                     5 or 6 slices), or the scalars run in launches of
  *                     their own (0); the results are the same bit for bit;
- *   "fft_form":       1, 0, 2 or 3: the split-form FFT (Nphi = r0 2^k,
- *                     2^k > L; default where the length has it), the
- *                     mixed-radix Stockham FFT, the pruned real DFT as one
+ *   "fft_form":       1, 0, 2 or 3: the default by length (the split-form
+ *                     FFT where Nphi = r0 2^k, 2^k > L, and Nphi >= 384; the
+ *                     mixed-radix FFT where its radices are 2 and 3, or up
+ *                     to 13, and L is large; a folded real DFT on FP64 MFMA
+ *                     otherwise), the mixed-radix Stockham FFT, the pruned
+ *                     real DFT as one
  *                     FP64 GEMM per direction against a cos/sin basis, or
  *                     the whole line as one chirp-z (Bluestein) convolution
  *                     of power-of-two length MP >= Nphi + 2L (MP <= 2048; any

@@ -14,7 +14,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libkemorin_sht.so")
 SOURCES = ["sht_plan.hip", "sht_legendre.hip", "sht_fft.hip", "sht_reorder.hip",
-           "sht_split.hip", "sht_capi.hip", "sht_batch.hip", "sht_pole.hip",
+           "sht_zfold.hip", "sht_split.hip", "sht_capi.hip", "sht_batch.hip", "sht_pole.hip",
            "sht_nonlinear.hip", "sht_copy.hip", "sht_coriolis.hip", "sht_tune.hip", "sht_dft.hip",
            "sht_files.hip"]
 ARCH = "gfx950"

@@ -1415,6 +1415,19 @@ static int launch_czt(sht_plan *p, int ncomp, bool bwd, const double *in, double
   return SHT_OK;
 }
 
+// Form 1 of a length: the folded DFT or an FFT (ns per line, backward):
+// split-form lengths: N = 192 0.75 / 1.21, N = 384 1.63 / 1.41;
+// radices 2 and 3: N = 1152 (L = 383) 8.9 / 9.3, N = 1536 14.9 / 10.8;
+// radices 5 to 13: N = 540 2.9 / 7.5, N = 1350 12.1 / 21.3, N = 2160
+// (L = 719) 27.9 / 38.3;
+// larger primes: N = 268 1.1 / 20.6, N = 1086 8.4 / 82.
+// The DFT grows as N L, the FFTs about as N: the lines lie between.
+static bool zfold_wins(const sht_plan *p) {
+  if (p->fft.fast) return p->nphi < 384;
+  if (p->fft.big) return true;
+  return p->L <= (p->fft_generic ? 800 : 400);
+}
+
 int fft_plan_init(sht_plan *p) {
   FftPlan &fp = p->fft;
   const int n = p->nphi;
@@ -1636,7 +1649,7 @@ int fft_plan_init(sht_plan *p) {
     }
 #undef KSHT_FFT3_ATTR
   }
-  return SHT_OK;
+  return zfold_wins(p) ? zfold_init(p) : SHT_OK;
 }
 
 #define KSHT_FFT3_CASE(K, NP, NCV, LDS, ...)                                                 \
@@ -1656,6 +1669,7 @@ static bool dft_applies(const sht_plan *p, const FourierAddr &xa) {
 int launch_fft_bwd(sht_plan *p, int ncomp, const double *X, FourierAddr xa, double *v) {
   if (dft_applies(p, xa)) return launch_dft_bwd(p, ncomp, X, xa, v);
   if (p->var_fft_form == 3 && p->fft.zm) return launch_czt(p, ncomp, true, X, v, xa);
+  if (p->var_fft_form == 1 && p->t.zfb) return launch_zfold(p, ncomp, true, X, v, xa);
   const long long nline = (long long)p->nr * p->nth;
   const int B = p->fft.lines_per_wg;
   const dim3 grid((unsigned)((nline + B - 1) / B), (unsigned)ncomp);
@@ -1696,6 +1710,7 @@ int launch_fft_bwd(sht_plan *p, int ncomp, const double *X, FourierAddr xa, doub
 int launch_fft_fwd(sht_plan *p, int ncomp, const double *v, double *X, FourierAddr xa) {
   if (dft_applies(p, xa)) return launch_dft_fwd(p, ncomp, v, X, xa);
   if (p->var_fft_form == 3 && p->fft.zm) return launch_czt(p, ncomp, false, v, X, xa);
+  if (p->var_fft_form == 1 && p->t.zfb) return launch_zfold(p, ncomp, false, v, X, xa);
   const long long nline = (long long)p->nr * p->nth;
   const int B = p->fft.lines_per_wg;
   const dim3 grid((unsigned)((nline + B - 1) / B), (unsigned)ncomp);

@@ -113,6 +113,7 @@ struct Tables {
   double2 *tw = nullptr;                        // FFT twiddles
   double2 *twn = nullptr;                       // exp(-2 pi i k / Nphi), k < Nphi
   double2 *ztab = nullptr;                      // chirp-z form: roots, filters, chirp
+  double *zfb = nullptr, *zff = nullptr;        // folded DFT tables, backward and forward
   long long *slot_off_X = nullptr, *slot_off_rtm = nullptr;  // 2L+1 each
   double *pole = nullptr;  // P_l^0, dP_l^1/dtheta at theta = 0 and pi, 4 (L+1)
 };
@@ -157,8 +158,8 @@ struct sht_plan {
   int var_bwd_fused = 1;
   // SHT_FLAG_CHECK_FINITE: device counter of non-finite outputs (else null)
   unsigned long long *nonfinite = nullptr;
-  // FFT form: 1 = split form n = r0 * 2^k where the plan has it, 0 = the
-  // mixed-radix Stockham form for every length, 2 = the pruned real DFT as an
+  // FFT form: 1 = by length (zfold_wins: split form n = r0 * 2^k, folded DFT
+  // or mixed radix), 0 = the mixed-radix Stockham form for every length, 2 = the pruned real DFT as an
   // FP64 GEMM (set-up on first selection: sht_dft.hip)
   int var_fft_form = 1;
   void *dft = nullptr;
@@ -259,6 +260,9 @@ int czt_init(sht_plan *p);
 void dft_free(sht_plan *p);
 int launch_dft_bwd(sht_plan *p, int ncomp, const double *X, FourierAddr xa, double *v);
 int launch_dft_fwd(sht_plan *p, int ncomp, const double *v, double *X, FourierAddr xa);
+// zonal transform as a folded DFT (sht_zfold.hip)
+int zfold_init(sht_plan *p);
+int launch_zfold(sht_plan *p, int ncomp, bool bwd, const double *in, double *out, FourierAddr xa);
 // reorders (sht_reorder.hip)
 int launch_zero_unused_rtp(sht_plan *p, int ncomp, double *rtp);
 int launch_rtm_to_rtp(sht_plan *p, int ncomp, const double *rtm, double *rtp);

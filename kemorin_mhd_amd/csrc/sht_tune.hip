@@ -7,9 +7,10 @@
 // fastest for the run.  Here the variants are the kernel forms of one plan:
 //   split_fwd_mfma  16 or 32: INT8 MFMA form of the forward split products
 //                   (split-precision plans);
-//   fft_form        1, 0, 2 or 3: split-form FFT (n = r0 2^k, where the
-//                   length has it), mixed-radix Stockham FFT, the pruned real
-//                   DFT as an FP64 GEMM (sht_dft.hip), or the whole line as
+//   fft_form        1, 0, 2 or 3: the default by length (split-form FFT,
+//                   folded DFT or mixed radix), mixed-radix Stockham FFT, the
+//                   pruned real DFT as an FP64 GEMM (sht_dft.hip), or the
+//                   whole line as
 //                   one chirp-z (Bluestein) convolution of power-of-two
 //                   length (sht_fft.hip).
 // Every combination runs one backward and one forward transform untimed,
@@ -139,9 +140,9 @@ extern "C" int sht_plan_autotune(sht_plan *p, int nvb, int nsb, int nvf, int nsf
       }
   }
   // candidate values of each knob that applies to this plan
-  std::vector<int> mfmas = {16}, forms = {p->fft.fast ? 1 : 0};
+  std::vector<int> mfmas = {16}, forms = {1};
   if (p->precision == SHT_PREC_SPLIT_INT8) mfmas.push_back(32);
-  if (p->fft.fast) forms.push_back(0);
+  if (p->fft.fast || p->t.zfb) forms.push_back(0);  // else form 1 is form 0
   if (dft_init(p) == SHT_OK) forms.push_back(2);  // the DFT product, where its set-up fits
   if (czt_init(p) == SHT_OK) forms.push_back(3);  // the chirp-z form, Nphi + 2L <= 2048
   const int keep_mfma = p->var_fwd_mfma, keep_form = p->var_fft_form;
