@@ -316,7 +316,7 @@ def run_engine(cfg, precision, args, torch, sp_b, grid_f, keep=False, otf=False,
     return dict(ms_per_step=ms, round_trips_per_s=1e3 / ms, timers=timers, plan_bytes=dev_bytes,
                 outputs=out, slices=(args.slices or 6) if precision == "split" else 0,
                 hbm_in_use_bytes=total_b - free_b, hbm_total_bytes=total_b, autotune=tuned,
-                bwd_fused=fused)
+                bwd_fused=fused, steps=args.steps)
 
 
 FIELDS_BWD = (("vector1", 0, 3), ("vector2", 3, 6), ("scalar1", 6, 7), ("scalar2", 7, 8))
@@ -409,17 +409,22 @@ def kernel_roofline(cfg_d, res, precision, slices):
             f"ksht::k_leg_bwd_split<{slices}, {4 if res.get('bwd_fused') else 3}, true>" if split
             else "ksht::k_leg_bwd<true>"),
         "legendre_forward_vector_kernel": (f"ksht::k_leg_fwd_split<{slices}, 3, true>" if split
-                                           else "ksht::k_leg_fwd<true>"),
+                                           else "ksht::k_leg_fwd"),
         "fft_backward": f"ksht::k_fft3_bwd<{npow}, 4>" if fast else "ksht::k_fft_bwd (mixed radix)",
         "fft_forward": f"ksht::k_fft3_fwd<{npow}, 8>" if fast else "ksht::k_fft_fwd (mixed radix)",
     }
     stages = {
-        "legendre_backward_vector_kernel": ("mfma", (12 if res.get("bwd_fused") else 10) * F1),
+        # the FP64 kernel takes vectors and scalars in one launch
+        "legendre_backward_vector_kernel": (
+            "mfma", (12 if res.get("bwd_fused") or not split else 10) * F1),
         "legendre_forward_vector_kernel": ("mfma", 15 * F1),
         "fft_backward": ("hbm", 8.0 * 8 * nline * (nslot + cfg_d["nphi"])),
         "fft_forward": ("hbm", 8.0 * 9 * nline * (nslot + cfg_d["nphi"])),
     }
     t = res["timers"]
+    # a stage of several launches per step (P tiles, packed shares) divides its
+    # work among them
+    stages = {s: (b, w / max(1.0, t[s][1] / res["steps"])) for s, (b, w) in stages.items()}
     avg = {s: t[s][0] / max(t[s][1], 1) for s in stages}
     dom = max(stages, key=lambda s: avg[s])
     bound, work = stages[dom]

@@ -109,6 +109,7 @@ struct Tables {
   double *Pb = nullptr, *dPb = nullptr, *Pf = nullptr, *dPf = nullptr;
   double *radius = nullptr, *a_r = nullptr;     // device, Nr
   double *weight = nullptr, *asin_t = nullptr;  // device, Ntheta
+  double2 *wt = nullptr;                        // (weight, 1/sin) of the hemisphere rows, padded
   double *cos_t = nullptr, *sin_t = nullptr;    // device, Ntheta
   double2 *tw = nullptr;                        // FFT twiddles
   double2 *twn = nullptr;                       // exp(-2 pi i k / Nphi), k < Nphi
@@ -140,6 +141,8 @@ struct sht_plan {
   bool fft_generic = false;  // FFT needs radices other than 2, 3, 4, 8
   double *X = nullptr;        // field-major Fourier workspace
   long long x_elems = 0;
+  double *Bp = nullptr;       // packed spectra of a backward call (FP64 products)
+  long long bp_elems = 0;
   long long device_bytes = 0;
   // split-precision state (allocated only in SHT_PREC_SPLIT_INT8 mode)
   void *split = nullptr;
@@ -244,6 +247,7 @@ void split_ws_bytes(const sht_plan *p, int ncomp, bool backward, long long *dig_
 int scratch_attach(int device);
 
 // Legendre launchers (sht_legendre.hip)
+int leg_init(sht_plan *p);
 int launch_leg_bwd(sht_plan *p, int nv, int ns, const double *sp, SpecAddr sa,
                    double *out, GridAddr ga);
 int launch_leg_fwd(sht_plan *p, int nv, int ns, const double *in, GridAddr ga,

@@ -357,7 +357,7 @@ static void free_plan(sht_plan *p) {
   if (!p) return;
   void *ptrs[] = {p->t.offb, p->t.offf, p->t.ipad, p->t.jst, p->t.Pb, p->t.dPb,
                   p->t.Pf, p->t.dPf, p->t.radius, p->t.a_r, p->t.weight, p->t.asin_t,
-                  p->t.cos_t, p->t.sin_t, p->t.tw, p->t.twn, p->t.ztab, p->t.zfb, p->t.zff, p->t.slot_off_X, p->t.slot_off_rtm,
+                  p->t.cos_t, p->t.sin_t, p->t.tw, p->t.twn, p->t.ztab, p->t.zfb, p->t.zff, p->Bp, p->t.wt, p->t.slot_off_X, p->t.slot_off_rtm,
                   p->t.pole, p->X, p->offb_r, p->offf_r, p->Pt, p->dPt, p->nonfinite};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
@@ -509,7 +509,7 @@ extern "C" int sht_plan_create(const sht_desc *d, sht_plan **out) {
     return SHT_ERR_OOM;
   }
   p->device_bytes += (long long)sizeof(double) * p->x_elems;
-  if (p->precision == SHT_PREC_SPLIT_INT8) CHECK(split_init(p));
+  CHECK(p->precision == SHT_PREC_SPLIT_INT8 ? split_init(p) : leg_init(p));
   if (hipStreamSynchronize(api_stream(p->stream)) != hipSuccess) {
     set_error("sht_plan_create: table generation failed: %s",
               hipGetErrorString(hipGetLastError()));
