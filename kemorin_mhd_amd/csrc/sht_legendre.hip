@@ -60,17 +60,8 @@ struct LegDims {
   int M0, nM, ncv, ncs;
   int ntv, nts;    // backward: row tiles of 16 (vectors) and 32 (scalars)
   unsigned nbv;    // work-groups of the vectors; the scalars' follow
-  int tpv, tps;    // forward: column tiles of a group of fields, and whether
-  bool flat_v, flat_s;  // it holds all of them
   int W;           // doubles per packed row
 };
-// the LDS-staged forward of the reference's rtm buffers
-struct LegDimsLds {
-  int L, nr, nth, nth_h, nth_hp, nv, ns, n_rt, ncg, nblk;
-  int M0, nM;
-};
-constexpr int kSclPer = 4;
-
 // sum over x = 1 .. n of ceil(x / u)
 __host__ __device__ inline long long ceil_sum(int n, int u) {
   const long long q = n / u, r = n % u;
@@ -458,18 +449,74 @@ __device__ __forceinline__ FwdRows fwd_rows(const LegDims &d, unsigned pitch, in
   return FwdRows{t * pitch, (d.nth - 1 - t) * pitch};
 }
 
-// Field and radius of element e of column tile ct; nf fields of step planes.
-// Flattened over all fields (tpg = all tiles) where the fields' planes lie
-// within 32-bit offsets of each other, else field by field.
+// Field and radius of element e of column tile ct among nf fields' columns.
 struct FwdCol {
   int q, k;
   bool ok;
 };
-__device__ __forceinline__ FwdCol fwd_col(const LegDims &d, int ct, int e, int nf, int tpg, bool flat) {
-  const int g = flat ? 0 : ct / tpg, i = (flat ? ct : ct - g * tpg) * 16 + e;
-  const int q = flat ? i / d.nr : 0;
-  const FwdCol c = {g + q, i - q * d.nr, i < (flat ? nf * d.nr : d.nr)};
-  return c.ok ? c : FwdCol{flat ? nf - 1 : g, d.nr - 1, false};
+__device__ __forceinline__ FwdCol fwd_col(const LegDims &d, int ct, int e, int nf) {
+  const int i = ct * 16 + e, q = i / d.nr;
+  const FwdCol c = {q, i - q * d.nr, i < nf * d.nr};
+  return c.ok ? c : FwdCol{nf - 1, d.nr - 1, false};
+}
+
+// spectra of a wave's vector tile: conjugate-slot terms, degree and radial factors
+__device__ __forceinline__ void fwd_vec_store(const LegDims &d, const d4 (&acc)[2][2][5], int M,
+                                              int i0, int ct, int lane, double *__restrict__ sp,
+                                              const SpecAddr &sa, const int *__restrict__ jst,
+                                              const double *__restrict__ radius) {
+  const int L = d.L, nsig = (M == 0) ? 1 : 2;
+  const int ii = i0 + (lane & 15);
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const FwdCol fr = fwd_col(d, ct, 4 * r + (lane >> 4), d.nv);
+    if (!fr.ok) continue;
+    const int qr = fr.q, kr = fr.k;
+    const double r1 = radius[kr], r2 = r1 * r1;
+#pragma unroll
+    for (int par = 0; par < 2; par++) {
+      const int l = M + 2 * ii + par;
+      if (l > L) continue;
+      const double g7 = g7_of(l, M);
+#pragma unroll
+      for (int sg = 0; sg < 2; sg++) {
+        if (sg >= nsig) continue;
+        const double ms = (sg == 0) ? (double)M : -(double)M;
+        double *o = sp + (long long)(jst[sg == 0 ? L + M : L - M] + l - M) * sa.s_j +
+                    (long long)kr * sa.s_k + (long long)(3 * qr) * sa.s_nd;
+        o[0] = r2 * g7 * acc[sg][par][0][r];
+        o[sa.s_nd] = r1 * g7 * (acc[sg][par][1][r] - ms * acc[sg][par][2][r]);
+        o[2 * sa.s_nd] = r1 * g7 * (-acc[sg][par][3][r] - ms * acc[sg][par][4][r]);
+      }
+    }
+  }
+}
+
+// spectra of a wave's scalar tile
+__device__ __forceinline__ void fwd_scl_store(const LegDims &d, const d4 (&acc)[2][2][2][2], int M,
+                                              int i0, int ct, int lane, double *__restrict__ sp,
+                                              const SpecAddr &sa, const int *__restrict__ jst) {
+  const int L = d.L, nsig = (M == 0) ? 1 : 2;
+#pragma unroll
+  for (int c = 0; c < 2; c++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      if (ct + c >= d.ncs) continue;
+      const FwdCol fr = fwd_col(d, ct + c, 4 * r + (lane >> 4), d.ns);
+      if (!fr.ok) continue;
+      const int qr = fr.q, kr = fr.k;
+      double *ok = sp + (long long)kr * sa.s_k + (long long)(3 * d.nv + qr) * sa.s_nd;
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int par = 0; par < 2; par++) {
+          const int l = M + 2 * (i0 + 16 * u + (lane & 15)) + par;
+          if (l > L) continue;
+          const double g6 = g6_of(l, M);
+          ok[(long long)(jst[L + M] + l - M) * sa.s_j] = g6 * acc[0][par][u][c][r];
+          if (nsig == 2) ok[(long long)(jst[L - M] + l - M) * sa.s_j] = g6 * acc[1][par][u][c][r];
+        }
+    }
 }
 
 // vectors: 16 pair indices of both parities, both slots: 20 products
@@ -485,10 +532,9 @@ __device__ __forceinline__ void leg_fwd_vec(
   const int ip0 = ipad[2 * M], ip1 = ipad[2 * M + 1];
   if (i0 >= ip0) return;
   const int nsig = (M == 0) ? 1 : 2;
-  const FwdCol fc = fwd_col(d, ct, lane & 15, d.nv, d.tpv, d.flat_v);
-  const int q0 = d.flat_v ? 0 : ct / d.tpv;  // uniform part of the field
-  const double *x = in + (long long)(3 * q0) * ga.s_nd;
-  const unsigned vx = (unsigned)(((fc.q - q0) * 3 * ga.s_nd + fc.k) * 8);
+  const FwdCol fc = fwd_col(d, ct, lane & 15, d.nv);
+  const double *x = in;
+  const unsigned vx = (unsigned)((fc.q * 3 * ga.s_nd + fc.k) * 8);
   const unsigned pitch = (unsigned)ga.s_t * 8;
   const long long so[2] = {ga.slot_off[L + M] * ga.slot_mul, ga.slot_off[L - M] * ga.slot_mul};
   // columns of P: an odd block may end before the even one (read the even
@@ -578,30 +624,7 @@ __device__ __forceinline__ void leg_fwd_vec(
     f0 = f1;
   }
   mul(f0, eq);
-  const int ii = i0 + (lane & 15);
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const FwdCol fr = fwd_col(d, ct, 4 * r + (lane >> 4), d.nv, d.tpv, d.flat_v);
-    if (!fr.ok) continue;
-    const int qr = fr.q, kr = fr.k;
-    const double r1 = radius[kr], r2 = r1 * r1;
-#pragma unroll
-    for (int par = 0; par < 2; par++) {
-      const int l = M + 2 * ii + par;
-      if (l > L) continue;
-      const double g7 = g7_of(l, M);
-#pragma unroll
-      for (int sg = 0; sg < 2; sg++) {
-        if (sg >= nsig) continue;
-        const double ms = (sg == 0) ? (double)M : -(double)M;
-        double *o = sp + (long long)(jst[sg == 0 ? L + M : L - M] + l - M) * sa.s_j +
-                    (long long)kr * sa.s_k + (long long)(3 * qr) * sa.s_nd;
-        o[0] = r2 * g7 * acc[sg][par][0][r];
-        o[sa.s_nd] = r1 * g7 * (acc[sg][par][1][r] - ms * acc[sg][par][2][r]);
-        o[2 * sa.s_nd] = r1 * g7 * (-acc[sg][par][3][r] - ms * acc[sg][par][4][r]);
-      }
-    }
-  }
+  fwd_vec_store(d, acc, M, i0, ct, lane, sp, sa, jst, radius);
 }
 
 // scalars: 32 pair indices by two tiles of 16 columns: 16 products
@@ -622,10 +645,9 @@ __device__ __forceinline__ void leg_fwd_scl(
 #pragma unroll
   for (int c = 0; c < 2; c++) {
     const int cc = ct + c < d.ncs ? ct + c : d.ncs - 1;
-    const FwdCol fc = fwd_col(d, cc, lane & 15, d.ns, d.tps, d.flat_s);
-    const int q0 = d.flat_s ? 0 : cc / d.tps;
-    x[c] = in + (long long)(3 * d.nv + q0) * ga.s_nd;
-    vx[c] = (unsigned)(((fc.q - q0) * ga.s_nd + fc.k) * 8);
+    const FwdCol fc = fwd_col(d, cc, lane & 15, d.ns);
+    x[c] = in + (long long)(3 * d.nv) * ga.s_nd;
+    vx[c] = (unsigned)((fc.q * ga.s_nd + fc.k) * 8);
   }
   const long long so[2] = {ga.slot_off[L + M] * ga.slot_mul, ga.slot_off[L - M] * ga.slot_mul};
   // columns of P, 32 of them: clamped to the block (products not stored)
@@ -696,26 +718,7 @@ __device__ __forceinline__ void leg_fwd_scl(
     f0 = f1;
   }
   mul(f0, eq);
-#pragma unroll
-  for (int c = 0; c < 2; c++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      if (ct + c >= d.ncs) continue;
-      const FwdCol fr = fwd_col(d, ct + c, 4 * r + (lane >> 4), d.ns, d.tps, d.flat_s);
-      if (!fr.ok) continue;
-      const int qr = fr.q, kr = fr.k;
-      double *ok = sp + (long long)kr * sa.s_k + (long long)(3 * d.nv + qr) * sa.s_nd;
-#pragma unroll
-      for (int u = 0; u < 2; u++)
-#pragma unroll
-        for (int par = 0; par < 2; par++) {
-          const int l = M + 2 * (i0 + 16 * u + (lane & 15)) + par;
-          if (l > L) continue;
-          const double g6 = g6_of(l, M);
-          ok[(long long)(jst[L + M] + l - M) * sa.s_j] = g6 * acc[0][par][u][c][r];
-          if (nsig == 2) ok[(long long)(jst[L - M] + l - M) * sa.s_j] = g6 * acc[1][par][u][c][r];
-        }
-    }
+  fwd_scl_store(d, acc, M, i0, ct, lane, sp, sa, jst);
 }
 
 // One launch for all fields: a work-group's waves take consecutive tiles of
@@ -743,193 +746,272 @@ __global__ void __launch_bounds__(256, 2) k_leg_fwd(
 }
 
 // ---------------------------------------------------------------------------
-// Forward of the reference's rtm buffers, radius slowest, whose rows have to
-// be transposed through LDS.  Work-group = (M, radius tile,
-// component group, degree block); 4 waves, wave w owns pair indices
-// i in [64*ib + 16*w, +16) of both parities (l = M + 2i + parity).  The
-// reduction runs over hemisphere rows in chunks of 16 staged in LDS as
-// weighted symmetric / antisymmetric combinations of the mirrored rows; the
-// rows of chunk tc+1 and the P/dP fragments are prefetched into registers
-// while chunk tc is reduced.
-template <bool VEC>
-__global__ void __launch_bounds__(256) k_leg_fwd_lds(
-    LegDimsLds d, int cg0, const double *__restrict__ in, GridAddr ga, double *__restrict__ sp,
-    SpecAddr sa, const int *__restrict__ jst, const long long *__restrict__ offf,
+// Forward, staged: a work-group's rows in LDS, as weighted symmetric and
+// antisymmetric combinations, once for its four waves instead of once a wave.
+// A wave then reads 4 fragments of P a K step from global memory where the
+// direct form reads 16 (rows that start anywhere in a line cost two L1
+// accesses each), and the combinations' FP64 operations, which take the
+// matrix unit's time, are shared.
+//
+// NT waves along the pair indices by NC = 4 / NT along the columns, as the
+// tiles of an order divide: groups of four tiles (NT = 4), then a remainder of
+// two and of one, so that no wave idles.  A chunk is 4 NT rows of 16 NC
+// columns, one (row, column) per thread, in two LDS buffers; the rows of the
+// next chunk travel while this one is multiplied.
+constexpr int kFwdWaves = 4, kPlane = 64 * kFwdWaves;  // doubles of a staged component: 4 NT x 16 NC
+
+// sum over y = 0 .. n of floor(y / D)
+__host__ __device__ inline int floor_sum(int n, int D) {
+  const int q = (n + 1) / D, r = (n + 1) % D;
+  return D * (q * (q - 1) / 2) + q * r;
+}
+// Tiles of U degrees of the orders with n, n - 8, n - 16, ... degrees: those
+// of one XCD (8 divides U, so that floor((n + U - 1 - 8 j) / U) counts eighths).
+template <int U>
+__host__ __device__ inline int xcd_tiles(int n) {
+  return n <= 0 ? 0 : floor_sum((n + U - 1) / 8, U / 8);
+}
+// Work-group b of a launch, eight classes of orders M0 + x, M0 + x + 8, ...
+// dealt to the XCDs: all tiles of four columns tiles in turn, so that the
+// groups that read the same rows run side by side on one L2.  An order of c
+// tiles has c work-groups per four column tiles.
+struct FwdGroup {
+  int M, c, sc, r;  // order (-1: none), its tiles, column block, group within it
+};
+template <int U>
+__device__ __forceinline__ FwdGroup fwd_group(const LegDims &d, unsigned b, int nsc) {
+  const int x = b & 7, i = (int)(b >> 3), n = d.L + 1 - d.M0 - x;
+  if (x >= d.nM) return FwdGroup{-1, 0, 0, 0};
+  const int all = xcd_tiles<U>(n);
+  int lo = 0, hi = (d.nM - 1 - x) / 8;
+  while (lo < hi) {  // the last order that starts at or before i
+    const int mid = (lo + hi + 1) / 2;
+    if ((all - xcd_tiles<U>(n - 8 * mid)) * nsc <= i)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  const int c = (n - 8 * lo + U - 1) / U, in = i - (all - xcd_tiles<U>(n - 8 * lo)) * nsc;
+  if (in >= c * nsc) return FwdGroup{-1, 0, 0, 0};
+  return FwdGroup{d.M0 + x + 8 * lo, c, in / c, in % c};
+}
+
+// LDS position of a chunk's (column tile, row, column).  Rows of radius-slowest
+// input are written along the colatitude: the columns of a row are permuted so
+// that neither that nor the fragments' reads meet in a bank.
+template <bool KFAST, int NT>
+__device__ __forceinline__ int stage_pos(int ctl, int row, int col) {
+  return (ctl * 4 * NT + row) * 16 + (KFAST ? col : col ^ (row & 15));
+}
+
+// VEC: components (r, t, p) of a tile of columns; else two tiles of scalars
+template <bool VEC, bool KFAST, int NT>
+__device__ __forceinline__ void leg_fwd_staged(
+    const LegDims &d, const FwdGroup &fg, double *__restrict__ lds,
+    const double *__restrict__ in, const GridAddr &ga, double *__restrict__ sp,
+    const SpecAddr &sa, const int *__restrict__ jst, const long long *__restrict__ offf,
     const int *__restrict__ ipad, const double *__restrict__ Pf,
     const double *__restrict__ dPf, const double *__restrict__ radius,
-    const double *__restrict__ weight, const double *__restrict__ asin_t) {
-  constexpr int NC = VEC ? 3 : kSclPer;
-  constexpr int NQ = VEC ? 5 : kSclPer;
-  constexpr int NU = NC * 2;  // staging items per thread: 2 sig x NC x 256 / 256
-  constexpr int SBUF = 2 * NC * 2 * 256;
-  __shared__ double sA[2][SBUF];  // [buf][sig][f][sym/asym][tt][kk]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // logical id = ((ib (L+1) + M) n_rt + rt) ncg + cgl in runs of one (M, row
-  // block) per XCD (xcd_group_order), sharing the P rows on one L2; the run
-  // index ib (L+1) + M puts consecutive orders on consecutive XCDs (row
-  // blocks past the degrees of M are empty, and the work of row block ib
-  // would otherwise all land on two XCDs)
-  long long b = xcd_group_order(blockIdx.x, gridDim.x, (long long)d.n_rt * d.ncg);
-  const int cgl = (int)(b % d.ncg);
-  b /= d.ncg;
-  const int rt = (int)(b % d.n_rt);
-  b /= d.n_rt;
-  const int M = d.M0 + (int)(b % d.nM);
-  const int ib = (int)(b / d.nM);
-  const int L = d.L;
+    const double2 *__restrict__ wt) {
+  constexpr int NC = kFwdWaves / NT, R = 4 * NT, NX = VEC ? 3 : 2;
+  constexpr int kBuf = 4 * NX * kPlane;
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_of_group();
+  const int L = d.L, M = fg.M, c4 = fg.c / 4;
+  const int ctl = wave / NT;
+  // groups of four tiles first, then those of two and of one
+  const int cg = NT == 4 ? fg.sc * 4 + fg.r / c4 : NT == 2 ? fg.sc * 2 + (fg.r & 1) : fg.sc;
+  const int i0 = ((NT == 4 ? fg.r % c4 * 4 : NT == 2 ? 4 * c4 : fg.c - 1) + wave % NT) * (VEC ? 16 : 32);
+  if (cg * NC >= (VEC ? d.ncv : (d.ncs + 1) / 2)) return;
   const int ip0 = ipad[2 * M], ip1 = ipad[2 * M + 1];
-  if (ib * 64 >= ip0) return;  // whole work-group beyond the degrees of M
-  const int nsig = (M == 0) ? 1 : 2;
-  const int k0 = rt * 16;
-  const int i0 = ib * 64 + wave * 16;
-  const bool active = i0 < ip0;
-  const int cg = cg0 + cgl;
-  const int nc = VEC ? 3 : min(kSclPer, d.ns - kSclPer * (cg - d.nv));
-  const int nd0 = VEC ? 3 * cg : 3 * d.nv + kSclPer * (cg - d.nv);
-  const long long of0 = offf[2 * M], of1 = offf[2 * M + 1];
-  const int slot0 = L + M, slot1 = L - M;
-  const bool odd_nth = (d.nth & 1) != 0;
-  const int t_eq = odd_nth ? d.nth / 2 : -1;
+  const long long so[2] = {ga.slot_off[L + M] * ga.slot_mul, ga.slot_off[L - M] * ga.slot_mul};
 
-  d4 acc[2][2][NQ];
+  // this thread's row and column(s)
+  const int srow = KFAST ? (tid >> 4) % R : tid % R, scol = KFAST ? tid & 15 : (tid / R) & 15;
+  const int sct = tid / (16 * R);
+  const double *xs[VEC ? 1 : 2];
+#pragma unroll
+  for (int j = 0; j < (VEC ? 1 : 2); j++) {
+    const int nf = VEC ? d.nv : d.ns;
+    int c = VEC ? (cg * NC + sct) * 16 + scol : ((cg * NC + sct) * 2 + j) * 16 + scol;
+    c = c < nf * d.nr ? c : nf * d.nr - 1;
+    const int q = c / d.nr, k = c - q * d.nr;
+    xs[j] = in + (VEC ? 3 * q : 3 * d.nv + q) * ga.s_nd + k * ga.s_k;
+  }
+  const int spos = stage_pos<KFAST, NT>(sct, srow, scol);
+  const unsigned pitch = (unsigned)ga.s_t * 8;
+  // pair y of the chunk's rows: slot y / NX, component y % NX
+  double xn[2 * NX], xm[2 * NX];
+  double2 xw;
+  bool xeq;
+  unsigned on = 0, os = 0;  // its rows of the chunk, bytes
+  auto stage_rows = [&](int c) {
+    const int i = c * R + srow, t = i < d.nth_h ? i : d.nth_h - 1;
+    on = (unsigned)t * pitch;
+    os = (unsigned)(d.nth - 1 - t) * pitch;
+    xw = wt[i];  // 0 past the equator
+    xeq = 2 * t + 1 == d.nth;
+  };
+  auto stage_load = [&](int y) {
+    const int sg = y / NX, f = y % NX;
+    const double *x = xs[VEC ? 0 : f] + so[sg] + (VEC ? f * ga.s_nd : 0);
+    xn[y] = ldu(x, on);
+    xm[y] = ldu(x, os);
+  };
+  auto stage_store = [&](double *buf, int y) {
+    const double z = xeq ? 0.0 : xm[y];
+    double *o = buf + 2 * y * kPlane + spos;
+    o[0] = (xn[y] + z) * xw.x;
+    o[kPlane] = xeq ? 0.0 : (xn[y] - z) * xw.x;
+    if (VEC && y == 0 && scol == 0 && sct == 0) buf[kBuf + srow] = xw.y;
+  };
+  // columns of P: an odd block may end before the even one (read what is
+  // there: its products are not stored), and a scalar tile's second half with
+  // it.  Planes: P and dP of both parities, or P of both halves.
+  const bool has_o = VEC ? i0 < ip1 : ip1 > 0;
+  const int ipo = has_o ? ip1 : ip0;
+  const long long oe = offf[2 * M], oo = has_o ? offf[2 * M + 1] : oe;
+  const double *p1 = VEC ? dPf : Pf;
+  unsigned ve[2], vo[2];
+#pragma unroll
+  for (int r = 0; r < 2; r++) {
+    const int i = VEC ? i0 : i0 + 16 * r;
+    ve[r] = (unsigned)(((lane >> 4) * ip0 + (i < ip0 ? i : 0) + (lane & 15)) * 8);
+    vo[r] = (unsigned)(((lane >> 4) * ipo + (i < ipo ? i : 0) + (lane & 15)) * 8);
+  }
+  struct Step {
+    double a[2][2];
+  };
+  auto pload = [&](int s, Step &f) {
+    f.a[0][0] = ldu(Pf + oe + 4LL * s * ip0, ve[0]);
+    f.a[0][1] = ldu(p1 + oe + 4LL * s * ip0, ve[1]);
+    f.a[1][0] = ldu(Pf + oo + 4LL * s * ipo, vo[0]);
+    f.a[1][1] = ldu(p1 + oo + 4LL * s * ipo, vo[1]);
+  };
+
+  constexpr int NA = VEC ? 5 : 4;
+  d4 acc[2][2][NA];
 #pragma unroll
   for (int s = 0; s < 2; s++)
 #pragma unroll
-    for (int p = 0; p < 2; p++)
+    for (int u = 0; u < 2; u++)
 #pragma unroll
-      for (int q = 0; q < NQ; q++) acc[s][p][q] = d4{0.0, 0.0, 0.0, 0.0};
-
-  double vn[NU], vs[NU];
-  auto stage_load = [&](int tc) {
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      const int idx = tid + 256 * u;
-      const int kk = idx & 15, tt = (idx >> 4) & 15, f = (idx >> 8) % NC, sg = idx / (256 * NC);
-      const int t = tc * 16 + tt, k = k0 + kk;
-      const bool valid = sg < nsig && f < nc && t < d.nth_h && k < d.nr;
-      const long long base = ga.slot_off[sg == 0 ? slot0 : slot1] * ga.slot_mul +
-                             (long long)(nd0 + f) * ga.s_nd + (long long)k * ga.s_k;
-      vn[u] = valid ? in[base + (long long)t * ga.s_t] : 0.0;
-      vs[u] = (valid && t != t_eq) ? in[base + (long long)(d.nth - 1 - t) * ga.s_t] : 0.0;
+      for (int c = 0; c < NA; c++) acc[s][u][c] = d4{0.0, 0.0, 0.0, 0.0};
+  auto mul = [&](const Step &f, const double *buf, int s) {
+    const double *x = buf + stage_pos<KFAST, NT>(ctl, 4 * s + (lane >> 4), lane & 15);
+    double ps[2];
+    if (VEC) {
+      const double as = buf[kBuf + 4 * s + (lane >> 4)];
+      ps[0] = f.a[0][0] * as;
+      ps[1] = f.a[1][0] * as;
     }
-  };
-  auto stage_store = [&](int tc, double *buf) {
 #pragma unroll
-    for (int u = 0; u < NU; u++) {
-      const int idx = tid + 256 * u;
-      const int kk = idx & 15, tt = (idx >> 4) & 15, f = (idx >> 8) % NC, sg = idx / (256 * NC);
-      const int t = tc * 16 + tt;
-      const double w = t < d.nth_h ? weight[t] : 0.0;
-      double *dst = buf + (((sg * NC + f) * 2) * 16 + tt) * 16 + kk;
-      dst[0] = (vn[u] + vs[u]) * w;
-      dst[256] = (t == t_eq) ? 0.0 : (vn[u] - vs[u]) * w;
-    }
-  };
-  double pc[4][2], dpc[4][2], pn[4][2], dpn[4][2], asc[4], asn_[4];
-  auto pload = [&](int tc, double (&a)[4][2], double (&da)[4][2], double (&as)[4]) {
+    for (int sg = 0; sg < 2; sg++)
 #pragma unroll
-    for (int ks = 0; ks < 4; ks++) {
-      const int t = tc * 16 + ks * 4 + (lane >> 4);
-      const long long c = i0 + (lane & 15);
-      const bool v1 = i0 < ip1;
-      a[ks][0] = Pf[of0 + (long long)t * ip0 + c];
-      a[ks][1] = v1 ? Pf[of1 + (long long)t * ip1 + c] : 0.0;
-      da[ks][0] = VEC ? dPf[of0 + (long long)t * ip0 + c] : 0.0;
-      da[ks][1] = (VEC && v1) ? dPf[of1 + (long long)t * ip1 + c] : 0.0;
-      as[ks] = (VEC && t < d.nth_h) ? asin_t[t] : 0.0;
-    }
-  };
-
-  const int nchunk = (d.nth_h + 15) / 16;
-  stage_load(0);
-  if (active) pload(0, pc, dpc, asc);
-  for (int tc = 0; tc < nchunk; tc++) {
-    double *buf = sA[tc & 1];
-    stage_store(tc, buf);
-    __syncthreads();
-    const bool more = tc + 1 < nchunk;
-    if (more) {
-      stage_load(tc + 1);
-      if (active) pload(tc + 1, pn, dpn, asn_);
-    }
-    if (active) {
+      for (int c = 0; c < NX; c++) {
+        const double u = x[(sg * NX + c) * 2 * kPlane];            // symmetric
+        const double v = x[((sg * NX + c) * 2 + 1) * kPlane];      // antisymmetric
+        if (!VEC) {
 #pragma unroll
-      for (int ks = 0; ks < 4; ks++) {
-        const int tt = ks * 4 + (lane >> 4);
-        const double asn = asc[ks];
-#pragma unroll
-        for (int par = 0; par < 2; par++) {
-          if (i0 >= (par ? ip1 : ip0)) continue;
-          const double bP = pc[ks][par], bdP = dpc[ks][par];
-          const int sP = par, sdP = 1 - par;  // P: sym for even, dP: asym for even
-#pragma unroll
-          for (int sg = 0; sg < 2; sg++) {
-            if (sg >= nsig) continue;
-            const int sc = (nsig == 1) ? 0 : 1 - sg;
-            const double *aa = buf + ((sg * NC * 2) * 16 + tt) * 16 + (lane & 15);
-            const double *ac = buf + ((sc * NC * 2) * 16 + tt) * 16 + (lane & 15);
-            if (VEC) {
-              const double avr = aa[(0 * 2 + sP) * 256];
-              const double avt = aa[(1 * 2 + sdP) * 256];
-              const double avp = aa[(2 * 2 + sdP) * 256];
-              const double avpc = ac[(2 * 2 + sP) * 256] * asn;
-              const double avtc = ac[(1 * 2 + sP) * 256] * asn;
-              acc[sg][par][0] = mfma64(avr, bP, acc[sg][par][0]);
-              acc[sg][par][1] = mfma64(avt, bdP, acc[sg][par][1]);
-              acc[sg][par][2] = mfma64(avpc, bP, acc[sg][par][2]);
-              acc[sg][par][3] = mfma64(avp, bdP, acc[sg][par][3]);
-              acc[sg][par][4] = mfma64(avtc, bP, acc[sg][par][4]);
-            } else {
-#pragma unroll
-              for (int c = 0; c < NQ; c++)
-                if (c < nc) acc[sg][par][c] = mfma64(aa[(c * 2 + sP) * 256], bP, acc[sg][par][c]);
-            }
+          for (int r = 0; r < 2; r++) {
+            acc[sg][0][2 * r + c] = mfma64(u, f.a[0][r], acc[sg][0][2 * r + c]);
+            acc[sg][1][2 * r + c] = mfma64(v, f.a[1][r], acc[sg][1][2 * r + c]);
           }
-        }
-      }
-    }
-    if (more && active) {
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++) {
-        asc[ks] = asn_[ks];
-#pragma unroll
-        for (int par = 0; par < 2; par++) {
-          pc[ks][par] = pn[ks][par];
-          dpc[ks][par] = dpn[ks][par];
-        }
-      }
-    }
-  }
-  if (!active) return;
-  const int ii = i0 + (lane & 15);
-#pragma unroll
-  for (int par = 0; par < 2; par++) {
-    const int l = M + 2 * ii + par;
-    if (l > L) continue;
-    const double g7 = g7_of(l, M), g6 = g6_of(l, M);
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int k = k0 + 4 * r + (lane >> 4);
-      if (k >= d.nr) continue;
-      const double r1 = radius[k], r2 = r1 * r1;
-#pragma unroll
-      for (int sg = 0; sg < 2; sg++) {
-        if (sg >= nsig) continue;
-        const double ms = (sg == 0) ? (double)M : -(double)M;
-        const long long o = (long long)(jst[sg == 0 ? slot0 : slot1] + l - M) * sa.s_j +
-                            (long long)k * sa.s_k + (long long)nd0 * sa.s_nd;
-        if (VEC) {
-          sp[o] = r2 * g7 * acc[sg][par][0][r];
-          sp[o + sa.s_nd] = r1 * g7 * (acc[sg][par][1][r] - ms * acc[sg][par][2][r]);
-          sp[o + 2 * sa.s_nd] = r1 * g7 * (-acc[sg][par][3][r] - ms * acc[sg][par][4][r]);
+        } else if (c == 0) {
+          acc[sg][0][0] = mfma64(u, f.a[0][0], acc[sg][0][0]);
+          acc[sg][1][0] = mfma64(v, f.a[1][0], acc[sg][1][0]);
         } else {
-#pragma unroll
-          for (int c = 0; c < NQ; c++)
-            if (c < nc) sp[o + (long long)c * sa.s_nd] = g6 * acc[sg][par][c][r];
+          // v_t: dP own slot (1), P / sin conjugate slot (4); v_p: 3 and 2
+          const int o = c == 1 ? 1 : 3, z = c == 1 ? 4 : 2;
+          acc[sg][0][o] = mfma64(v, f.a[0][1], acc[sg][0][o]);
+          acc[sg][1][o] = mfma64(u, f.a[1][1], acc[sg][1][o]);
+          acc[1 - sg][0][z] = mfma64(u, ps[0], acc[1 - sg][0][z]);
+          acc[1 - sg][1][z] = mfma64(v, ps[1], acc[1 - sg][1][z]);
         }
+      }
+  };
+  const int nstep = (d.nth_h + 3) / 4, last = nstep - 1;
+  constexpr int kPitch = kBuf + 16;  // a buffer and 1/sin of its rows
+  Step f[4];
+  pload(0, f[0]);
+  pload(last < 1 ? last : 1, f[1]);
+  stage_rows(0);
+#pragma unroll
+  for (int y = 0; y < 2 * NX; y++) stage_load(y);
+#pragma unroll
+  for (int y = 0; y < 2 * NX; y++) stage_store(lds, y);
+  __syncthreads();
+  // P two steps ahead; the pairs of the next chunk a few per step, each
+  // written two steps after its load where the chunk has four
+  constexpr int kPer = NT == 4 ? (2 * NX + 2) / 3 : 2 * NX;
+  int cur = 0;
+  for (int q = 0; q < nstep; q += 4) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const int st = q + s, sc = s % NT;
+      if (st >= nstep) break;
+      const double *buf = lds + cur;
+      double *nxt = lds + (kPitch - cur);
+      pload(st + 2 < nstep ? st + 2 : last, f[(s + 2) & 3]);
+      if (sc == 0) stage_rows(st + NT < nstep ? st / NT + 1 : 0);
+#pragma unroll
+      for (int y = sc * kPer; y < (sc + 1) * kPer && y < 2 * NX; y++) stage_load(y);
+      __builtin_amdgcn_sched_barrier(0);
+      mul(f[s], buf, sc);
+      __builtin_amdgcn_sched_barrier(0);
+      // pairs loaded a step ago (all of them at the end of a shorter chunk)
+#pragma unroll
+      for (int y = NT == 4 ? (sc - 1) * kPer : sc == NT - 1 ? 0 : 2 * NX;
+           y < (NT == 4 ? sc * kPer : 2 * NX) && y < 2 * NX; y++)
+        if (y >= 0) stage_store(nxt, y);
+      if (sc == NT - 1) {
+        __syncthreads();
+        cur = kPitch - cur;
       }
     }
   }
+  if constexpr (VEC) {
+    fwd_vec_store(d, acc, M, i0, cg * NC + ctl, lane, sp, sa, jst, radius);
+  } else {
+    d4 q[2][2][2][2];
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+      q[i >> 3][(i >> 2) & 1][(i >> 1) & 1][i & 1] = acc[i >> 3][(i >> 2) & 1][i & 3];
+    fwd_scl_store(d, q, M, i0, (cg * NC + ctl) * 2, lane, sp, sa, jst);
+  }
+}
+
+// One launch for all fields: the scalars' work-groups follow the vectors'.
+template <bool KFAST>
+__global__ void __launch_bounds__(64 * kFwdWaves, 2) k_leg_fwd_lds(
+    LegDims d, const double *__restrict__ in, GridAddr ga, double *__restrict__ sp, SpecAddr sa,
+    const int *__restrict__ jst, const long long *__restrict__ offf,
+    const int *__restrict__ ipad, const double *__restrict__ Pf,
+    const double *__restrict__ dPf, const double *__restrict__ radius,
+    const double2 *__restrict__ wt) {
+  __shared__ double lds[2 * (12 * kPlane + 16)];
+  const bool vec = blockIdx.x < d.nbv;
+  const FwdGroup g = vec ? fwd_group<32>(d, blockIdx.x, (d.ncv + kFwdWaves - 1) / kFwdWaves)
+                         : fwd_group<64>(d, blockIdx.x - d.nbv, ((d.ncs + 1) / 2 + kFwdWaves - 1) / kFwdWaves);
+  if (g.M < 0) return;
+  const int rest = g.r - (g.c & ~3);  // below 0: of a group of four
+#define KSHT_KIND(VEC, NT)                                                                       \
+  leg_fwd_staged<VEC, KFAST, NT>(d, g, lds, in, ga, sp, sa, jst, offf, ipad, Pf, dPf, radius, wt)
+  if (vec) {
+    if (rest < 0)
+      KSHT_KIND(true, 4);
+    else if ((g.c & 2) && rest < 2)
+      KSHT_KIND(true, 2);
+    else
+      KSHT_KIND(true, 1);
+  } else {
+    if (rest < 0)
+      KSHT_KIND(false, 4);
+    else if ((g.c & 2) && rest < 2)
+      KSHT_KIND(false, 2);
+    else
+      KSHT_KIND(false, 1);
+  }
+#undef KSHT_KIND
 }
 
 // Packed spectra: all orders of a call up to 1 GiB, else that much of them at
@@ -976,8 +1058,6 @@ static LegDims make_dims(const sht_plan *p, int nv, int ns) {
   d.ntv = (p->nth_h + 15) / 16;
   d.nts = (p->nth_h + 31) / 32;
   d.nbv = 0;
-  d.tpv = d.tps = 1;
-  d.flat_v = d.flat_s = true;
   d.W = 2 * 16 * (3 * d.ncv + d.ncs);
   return d;
 }
@@ -1039,70 +1119,53 @@ int launch_leg_bwd(sht_plan *p, int nv, int ns, const double *sp, SpecAddr sa, d
   return SHT_OK;
 }
 
-static int launch_leg_fwd_lds(sht_plan *p, const PTile &pt, int nv, int ns, const double *in,
-                              GridAddr ga, double *sp, SpecAddr sa) {
-  LegDimsLds d;
-  d.L = p->L;
-  d.nr = p->nr;
-  d.nth = p->nth;
-  d.nth_h = p->nth_h;
-  d.nth_hp = p->nth_hp;
-  d.nv = nv;
-  d.ns = ns;
-  d.n_rt = p->nr_p / 16;
-  d.nblk = ((p->L + 2) / 2 + 63) / 64;
-  d.M0 = pt.M0;
-  d.nM = pt.M1 - pt.M0;
-  const int nsg = (ns + kSclPer - 1) / kSclPer;
-  ForkJoin fj(p, nv > 0 && nsg > 0);  // scalar groups beside the vector groups
-  for (int vec = 1; vec >= 0; vec--) {
-    d.ncg = vec ? nv : nsg;
-    if (d.ncg == 0) continue;
-    const hipStream_t st = fj.stream(!vec);
-    const dim3 g((unsigned)((long long)d.nM * d.n_rt * d.ncg * d.nblk)), bl(256);
-    if (vec) {
-      StageTimer tk(p, 6);
-      hipLaunchKernelGGL(k_leg_fwd_lds<true>, g, bl, 0, st, d, 0, in, ga, sp, sa, p->t.jst,
-                         pt.offf, p->t.ipad, pt.Pf, pt.dPf, p->t.radius, p->t.weight, p->t.asin_t);
-    } else
-      hipLaunchKernelGGL(k_leg_fwd_lds<false>, g, bl, 0, st, d, nv, in, ga, sp, sa, p->t.jst,
-                         pt.offf, p->t.ipad, pt.Pf, pt.dPf, p->t.radius, p->t.weight, p->t.asin_t);
-    KSHT_HIP(hipGetLastError());
+// Staged from this many waves of a call on: it reads the rows once for four
+// waves but starts and ends them together.  Direct / staged: L = 127, 7
+// components, Nr = 65 (2900 waves) 137 / 147 us, L = 361, 4, Nr = 63 (11000)
+// 826 / 850, L = 255, 9, Nr = 129 (29000) 1590 / 1560, 18, Nr = 65 (29000)
+// 1750 / 1630.
+constexpr long long kFwdStaged = 16384;
+
+// work-groups of the staged forward: eight times the most of an XCD's orders
+template <int U>
+static unsigned fwd_groups(const LegDims &d, int nct) {
+  int most = 0;
+  for (int x = 0; x < 8 && x < d.nM; x++) {
+    const int n = d.L + 1 - d.M0 - x, j = (d.nM - 1 - x) / 8 + 1;
+    const int t = xcd_tiles<U>(n) - xcd_tiles<U>(n - 8 * j);
+    most = t > most ? t : most;
   }
-  return SHT_OK;
+  return 8u * (unsigned)most * (unsigned)((nct + kFwdWaves - 1) / kFwdWaves);
 }
 
 int launch_leg_fwd(sht_plan *p, int nv, int ns, const double *in, GridAddr ga, double *sp,
                    SpecAddr sa) {
   LegDims d = make_dims(p, nv, ns);
-  // the lanes of a flattened tile reach every field by a 32-bit offset
-  const long long lim = (1LL << 32) - 8LL * p->nr * p->nth, nd8 = 8 * ga.s_nd;
-  d.flat_v = 3LL * (nv - 1) * nd8 < lim;
-  d.flat_s = (ns - 1) * nd8 < lim;
-  const int tp1 = col_tiles(p, 1);
-  d.tpv = d.flat_v ? d.ncv : tp1;
-  d.tps = d.flat_s ? d.ncs : tp1;
-  if (!d.flat_v) d.ncv = nv * tp1;
-  if (!d.flat_s) d.ncs = ns * tp1;
-  const long long nct = (d.ncs + 1) / 2;
   for (int ti = 0; ti < ptile_count(p); ti++) {
     PTile pt;
     int rc = ptile_prepare(p, ti, true, &pt);
     if (rc) return rc;
-    if (ga.s_k != 1 || lim <= 0) {
-      if ((rc = launch_leg_fwd_lds(p, pt, nv, ns, in, ga, sp, sa))) return rc;
-      continue;
-    }
     StageTimer tk(p, 6);
     d.M0 = pt.M0;
     d.nM = pt.M1 - pt.M0;
+    // direct: the lanes of a flattened tile reach every field by a 32-bit offset
+    const long long lim = (1LL << 32) - 8LL * p->nr * p->nth, nd8 = 8 * ga.s_nd;
     d.ntv = (int)(ceil_sum(p->L + 1 - pt.M0, 32) - ceil_sum(p->L + 1 - pt.M1, 32));
     d.nts = (int)(ceil_sum(p->L + 1 - pt.M0, 64) - ceil_sum(p->L + 1 - pt.M1, 64));
-    const int nw = group_waves((long long)d.ntv * d.ncv + d.nts * nct);
-    d.nbv = groups(d.ntv, nw) * (unsigned)d.ncv;
-    const dim3 g(d.nbv + groups(d.nts, nw) * (unsigned)nct), bl(64 * nw);
-    hipLaunchKernelGGL(k_leg_fwd, g, bl, 0, p->stream, d, in, ga, sp, sa, p->t.jst, pt.offf,
-                       p->t.ipad, pt.Pf, pt.dPf, p->t.radius, p->t.wt);
+    const long long nct = (d.ncs + 1) / 2, waves = (long long)d.ntv * d.ncv + d.nts * nct;
+    if (ga.s_k == 1 && lim > 3LL * (nv - 1) * nd8 && lim > (ns - 1) * nd8 && waves < kFwdStaged) {
+      const int nw = group_waves(waves);
+      d.nbv = groups(d.ntv, nw) * (unsigned)d.ncv;
+      const dim3 g(d.nbv + groups(d.nts, nw) * (unsigned)nct), bl(64 * nw);
+      hipLaunchKernelGGL(k_leg_fwd, g, bl, 0, p->stream, d, in, ga, sp, sa, p->t.jst, pt.offf,
+                         p->t.ipad, pt.Pf, pt.dPf, p->t.radius, p->t.wt);
+    } else {
+      d.nbv = nv ? fwd_groups<32>(d, d.ncv) : 0;
+      const unsigned nb = d.nbv + (ns ? fwd_groups<64>(d, (int)nct) : 0);
+      const auto kern = ga.s_k == 1 ? k_leg_fwd_lds<true> : k_leg_fwd_lds<false>;
+      hipLaunchKernelGGL(kern, dim3(nb), dim3(64 * kFwdWaves), 0, p->stream, d, in, ga, sp, sa, p->t.jst,
+                         pt.offf, p->t.ipad, pt.Pf, pt.dPf, p->t.radius, p->t.wt);
+    }
     KSHT_HIP(hipGetLastError());
   }
   return SHT_OK;
