@@ -55,7 +55,9 @@ typedef struct {
   int nidx_phi;     /* Nphi: longitudes (even, > 2L+1)                   */
   const double *radius; /* host array of Nr radii                        */
   int max_ncomp;    /* largest ncomp a call will pass (workspace size)    */
-  int precision;    /* SHT_PREC_FP64 or SHT_PREC_SPLIT_INT8              */
+  int precision;    /* SHT_PREC_FP64 or SHT_PREC_SPLIT_INT8: products of  */
+                    /* INT8 slices where they are the faster ones (L from */
+                    /* 448 on; 5 slices 384, 4 slices 224), FP64 below    */
   int n_slices;     /* split mode: INT8 slices per operand (0 = default) */
   int flags;        /* SHT_FLAG_* bits, 0 for none                      */
 } sht_desc;
@@ -106,6 +108,11 @@ long long sht_plan_device_bytes(const sht_plan *plan);
  *                     whose product shares the vector's P slices (1, for
  *                     5 or 6 slices), or the scalars run in launches of
  *                     their own (0); the results are the same bit for bit;
+ *   "split_all":       0 (default) or 1: a split-precision plan runs FP64
+ *                     products below the truncations where sliced ones are
+ *                     faster (precision, above), or sliced ones at every size
+ *                     (their tables are set up, and counted in the plan's
+ *                     device bytes, when first selected);
  *   "fft_form":       1, 0, 2 or 3: the default by length (the split-form
  *                     FFT where Nphi = r0 2^k, 2^k > L, and Nphi >= 384; the
  *                     mixed-radix FFT where its radices are 2 and 3, or up
@@ -123,7 +130,7 @@ long long sht_plan_device_bytes(const sht_plan *plan);
 int sht_plan_set_variant(sht_plan *plan, const char *name, int value);
 int sht_plan_get_variant(const sht_plan *plan, const char *name, int *value);
 /* Tile-shape autotuner: times every applicable combination of the plan's
- * variants ("split_fwd_mfma" for split-precision plans, "fft_form" among the
+ * variants ("split_fwd_mfma" for plans on sliced products, "fft_form" among the
  * forms that apply to the length) on synthetic device data of the given field
  * sets (one backward of nvector_b/nscalar_b and one forward of
  * nvector_f/nscalar_f per round trip, best of three) and keeps the fastest.

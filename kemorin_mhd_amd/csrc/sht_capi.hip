@@ -74,14 +74,14 @@ static FourierAddr rtp_fourier_addr(const sht_plan *p, int ncomp) {
 static int leg_bwd(sht_plan *p, const Workspace &ws, int nv, int ns, const double *sp,
                    SpecAddr sa, double *out, GridAddr ga) {
   StageTimer tm(p, 0);
-  if (p->precision == SHT_PREC_SPLIT_INT8)
+  if (p->digits)
     return launch_leg_bwd_split(p, ws, nv, ns, sp, sa, out, ga);
   return launch_leg_bwd(p, nv, ns, sp, sa, out, ga);
 }
 static int leg_fwd(sht_plan *p, const Workspace &ws, int nv, int ns, const double *in,
                    GridAddr ga, double *sp, SpecAddr sa) {
   StageTimer tm(p, 3);
-  if (p->precision == SHT_PREC_SPLIT_INT8)
+  if (p->digits)
     return launch_leg_fwd_split(p, ws, nv, ns, in, ga, sp, sa);
   return launch_leg_fwd(p, nv, ns, in, ga, sp, sa);
 }

@@ -144,7 +144,9 @@ struct sht_plan {
   double *Bp = nullptr;       // packed spectra of a backward call (FP64 products)
   long long bp_elems = 0;
   long long device_bytes = 0;
-  // split-precision state (allocated only in SHT_PREC_SPLIT_INT8 mode)
+  // split-precision plans: whether the products run as sliced digits, and the
+  // state they need (split_init)
+  bool digits = false;
   void *split = nullptr;
   // P tables generated per call, one m-tile at a time, into tile buffers
   // (SHT_FLAG_P_ON_THE_FLY) instead of stored for all orders
@@ -159,6 +161,8 @@ struct sht_plan {
   // split backward: 1 = each vector group's launch also takes one scalar
   // (sharing its P slices), 0 = scalars in launches of their own
   int var_bwd_fused = 1;
+  // split-precision plans: 1 = sliced products at every size, 0 = split_wins
+  int var_split_all = 0;
   // SHT_FLAG_CHECK_FINITE: device counter of non-finite outputs (else null)
   unsigned long long *nonfinite = nullptr;
   // FFT form: 1 = by length (zfold_wins: split form n = r0 * 2^k, folded DFT
@@ -290,6 +294,19 @@ int pole_tables_init(sht_plan *p);
 // split precision (sht_split.hip)
 int split_init(sht_plan *p);
 void split_free(sht_plan *p);
+// Whether the sliced products of a split-precision plan beat its FP64 ones,
+// which need no slicing pass over the data.  Legendre stages, backward /
+// forward, sliced against FP64: 6 slices L = 127, Nr = 65, 8 and 7 components
+// 286 / 271 against 153 / 178 us, L = 255, 9 components 1098 / 1000 against
+// 822 / 795, L = 361, 4, Nr = 63 925 / 1071 against 824 / 826, L = 511, 8, Nr
+// = 65 4.07 / 4.66 against 4.04 / 4.46 ms, 9, Nr = 257 18.0 / 18.1 against
+// 17.8 / 18.2, L = 1023, 8 34.2 / 46.8 against 35.0 / 44.2.  5 slices, 9
+// components, Nr = 65: L = 255 957 / 885 us, L = 511 4.49 / 4.45 against 4.61
+// / 4.94 ms.  4 slices: L = 191 559 / 514 against 421 / 421 us, L = 255 814 /
+// 773.
+inline bool split_wins(int L, int n_slices) {
+  return L >= (n_slices >= 6 ? 448 : n_slices == 5 ? 384 : 224);
+}
 int launch_leg_bwd_split(sht_plan *p, const Workspace &ws, int nv, int ns, const double *sp,
                          SpecAddr sa, double *out, GridAddr ga);
 int launch_leg_fwd_split(sht_plan *p, const Workspace &ws, int nv, int ns, const double *in,

@@ -1023,21 +1023,41 @@ static long long pack_elems(const sht_plan *p, int W) {
   return all < cap ? all : one > cap ? one : cap;
 }
 
+// Packing pays once its launch (6 to 10 us) costs less than the waves lose
+// to scattered loads: L = 31, 8 components, Nr = 33 (416 waves) 14 us direct
+// against 8 + 11 packed, L = 63, 4, Nr = 17 (512) 18 / 10 + 13; L = 127, 7,
+// Nr = 65 (8000) 270 / 34 + 164, L = 361, 4, Nr = 63 (31000) 1400 / 130 + 720.
+// Spectra past the 32-bit offsets of the direct loads are packed always.
+static bool packs(const sht_plan *p, int nv, int ns) {
+  const long long waves =
+      (p->L + 1) * ((nv ? (long long)col_tiles(p, nv) * ((p->nth_h + 15) / 16) : 0) +
+                    (ns ? (long long)((col_tiles(p, ns) + 1) / 2) * ((p->nth_h + 31) / 32) : 0));
+  return waves >= 2048 || (3LL * nv + ns) * p->jmax * p->nr >= (1LL << 28);
+}
+
 int leg_init(sht_plan *p) {
-  // the widest rows of any call: max_ncomp scalars, or as many vectors
+  bool any = false;  // a call of the plan's that packs
+  for (int nv = 0; 3 * nv <= p->max_ncomp; nv++) any |= packs(p, nv, p->max_ncomp - 3 * nv);
+  // the widest rows of any call: max_ncomp scalars, or as many vectors; where
+  // memory is short, fewer orders at a time
   const int W = 2 * 16 * (col_tiles(p, p->max_ncomp) + 3);
-  p->bp_elems = pack_elems(p, W);
+  const long long one = pack_rows(p->L + 1) * W;
+  p->bp_elems = any ? pack_elems(p, W) : 0;
   std::vector<double2> wt(p->nth_hp, make_double2(0.0, 0.0));
   for (int t = 0; t < p->nth_h; t++) wt[t] = make_double2(p->weight[t], p->asin_t[t]);
-  const size_t bytes = sizeof(double) * (size_t)p->bp_elems, wb = sizeof(double2) * wt.size();
-  if (hipMalloc(&p->Bp, bytes) != hipSuccess) {
+  const size_t wb = sizeof(double2) * wt.size();
+  while (p->bp_elems && hipMalloc(&p->Bp, sizeof(double) * (size_t)p->bp_elems) != hipSuccess) {
     p->Bp = nullptr;
-    set_error("sht_plan_create: packed spectra of %zu bytes: out of device memory", bytes);
-    return SHT_ERR_OOM;
+    (void)hipGetLastError();
+    if (p->bp_elems == one) {
+      set_error("sht_plan_create: packed spectra of %lld bytes: out of device memory", 8 * one);
+      return SHT_ERR_OOM;
+    }
+    p->bp_elems = p->bp_elems / 4 > one ? p->bp_elems / 4 : one;
   }
   KSHT_HIP(hipMalloc(&p->t.wt, wb));
   KSHT_HIP(hipMemcpy(p->t.wt, wt.data(), wb, hipMemcpyHostToDevice));
-  p->device_bytes += (long long)(bytes + wb);
+  p->device_bytes += 8 * p->bp_elems + (long long)wb;
   return SHT_OK;
 }
 
@@ -1070,14 +1090,9 @@ static unsigned groups(long long waves, int nw) { return (unsigned)((waves + nw 
 int launch_leg_bwd(sht_plan *p, int nv, int ns, const double *sp, SpecAddr sa, double *out,
                    GridAddr ga) {
   LegDims d = make_dims(p, nv, ns);
-  const long long W = d.W, cap = p->bp_elems;
+  const long long W = d.W, cap = p->bp_elems > 0 ? p->bp_elems : 1;
   const long long per_v = (long long)d.ncv * d.ntv, per_s = (long long)((d.ncs + 1) / 2) * d.nts;
-  // Packing pays once its launch (6 to 10 us) costs less than the waves lose
-  // to scattered loads: L = 31, 8 components, Nr = 33 (416 waves) 14 us direct
-  // against 8 + 11 packed, L = 63, 4, Nr = 17 (512) 18 / 10 + 13; L = 127, 7,
-  // Nr = 65 (8000) 270 / 34 + 164, L = 361, 4, Nr = 63 (31000) 1400 / 130 + 720.
-  const bool pack = (p->L + 1) * (per_v + per_s) >= 2048 ||
-                    (long long)p->nr * sa.s_k >= (1LL << 28);
+  const bool pack = packs(p, nv, ns);
   int dt = 1;  // degrees of a packed run
   while (2 * dt * d.ncomp <= kPackRun) dt *= 2;
   for (int ti = 0; ti < ptile_count(p); ti++) {

@@ -509,7 +509,11 @@ extern "C" int sht_plan_create(const sht_desc *d, sht_plan **out) {
     return SHT_ERR_OOM;
   }
   p->device_bytes += (long long)sizeof(double) * p->x_elems;
-  CHECK(p->precision == SHT_PREC_SPLIT_INT8 ? split_init(p) : leg_init(p));
+  if (p->precision == SHT_PREC_SPLIT_INT8) {
+    if (p->n_slices == 0) p->n_slices = 6;
+    p->digits = split_wins(L, p->n_slices);
+  }
+  CHECK(p->digits ? split_init(p) : leg_init(p));
   if (hipStreamSynchronize(api_stream(p->stream)) != hipSuccess) {
     set_error("sht_plan_create: table generation failed: %s",
               hipGetErrorString(hipGetLastError()));
@@ -552,6 +556,11 @@ static int *variant_slot(sht_plan *p, const char *name, const int **allowed, int
     *nallowed = 2;
     return &p->var_bwd_fused;
   }
+  if (!strcmp(name, "split_all")) {
+    *allowed = onoff;
+    *nallowed = 2;
+    return &p->var_split_all;
+  }
   if (!strcmp(name, "fft_form")) {
     *allowed = form;
     *nallowed = 4;
@@ -579,7 +588,24 @@ extern "C" int sht_plan_set_variant(sht_plan *p, const char *name, int value) {
         const int rc = value == 2 ? dft_init(p) : czt_init(p);
         if (rc) return rc;
       }
+      if (slot == &p->var_split_all && value == 1 && p->precision == SHT_PREC_SPLIT_INT8 &&
+          !p->split) {
+        const long long bytes = p->device_bytes;
+        int rc = split_init(p);
+        if (!rc && hipStreamSynchronize(api_stream(p->stream)) != hipSuccess) {
+          set_error("sht_plan_set_variant: table slicing failed: %s",
+                    hipGetErrorString(hipGetLastError()));
+          rc = SHT_ERR_HIP;
+        }
+        if (rc) {
+          (void)hipGetLastError();
+          split_free(p);
+          p->device_bytes = bytes;
+          return rc;
+        }
+      }
       *slot = value;
+      p->digits = p->split && (p->var_split_all || split_wins(p->L, p->n_slices));
       return SHT_OK;
     }
   set_error("sht_plan_set_variant: %s = %d is not an allowed value", name, value);

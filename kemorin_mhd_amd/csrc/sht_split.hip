@@ -1686,7 +1686,7 @@ static int slice_tables(sht_plan *p, SplitState *st) {
 }
 
 int split_init(sht_plan *p) {
-  int S = p->n_slices == 0 ? 6 : p->n_slices;
+  const int S = p->n_slices;
   if (S < 4 || S > 7) {
     set_error("split precision: n_slices must be 4..7 (got %d)", p->n_slices);
     return SHT_ERR_ARG;
@@ -1694,7 +1694,6 @@ int split_init(sht_plan *p) {
   SplitState *st = new SplitState();
   st->S = S;
   p->split = st;
-  p->n_slices = S;
   int rc = table_layouts(p, st);
   if (rc) return rc;
   // the FP64 tables must be complete before slicing (same stream)
@@ -1725,10 +1724,14 @@ void split_free(sht_plan *p) {
 
 void split_ws_bytes(const sht_plan *p, int ncomp, bool backward, long long *dig_bytes,
                     long long *dexp_bytes) {
-  const SplitState *st = (const SplitState *)p->split;
-  const long long groups =
-      backward ? st->nchb * ncomp : (long long)p->nslot * st->nchf * 2 * ncomp;
-  *dig_bytes = groups * st->S * (p->nr_p / 16) * 1024;
+  // counted for every split-precision plan, whichever products it runs
+  long long nchb = 0;
+  for (int sl = 0; sl < p->nslot; sl++) {
+    const int M = sl >= p->L ? sl - p->L : p->L - sl, n = p->L - M + 1;
+    nchb += bchunk_count(M, (n + 1) / 2) + bchunk_count(M, n / 2);
+  }
+  const long long groups = backward ? nchb * ncomp : (long long)p->nslot * (p->nth_hp / 64) * 2 * ncomp;
+  *dig_bytes = groups * p->n_slices * (p->nr_p / 16) * 1024;
   *dexp_bytes = groups * p->nr_p * 4;
 }
 

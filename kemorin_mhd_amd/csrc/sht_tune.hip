@@ -141,7 +141,7 @@ extern "C" int sht_plan_autotune(sht_plan *p, int nvb, int nsb, int nvf, int nsf
   }
   // candidate values of each knob that applies to this plan
   std::vector<int> mfmas = {16}, forms = {1};
-  if (p->precision == SHT_PREC_SPLIT_INT8) mfmas.push_back(32);
+  if (p->digits) mfmas.push_back(32);
   if (p->fft.fast || p->t.zfb) forms.push_back(0);  // else form 1 is form 0
   if (dft_init(p) == SHT_OK) forms.push_back(2);  // the DFT product, where its set-up fits
   if (czt_init(p) == SHT_OK) forms.push_back(3);  // the chirp-z form, Nphi + 2L <= 2048
