@@ -111,6 +111,7 @@ struct Tables {
   double *weight = nullptr, *asin_t = nullptr;  // device, Ntheta
   double2 *wt = nullptr;                        // (weight, 1/sin) of the hemisphere rows, padded
   double *cos_t = nullptr, *sin_t = nullptr;    // device, Ntheta
+  double *sect = nullptr;                       // P per call: sectoral factors, L+2
   double2 *tw = nullptr;                        // FFT twiddles
   double2 *twn = nullptr;                       // exp(-2 pi i k / Nphi), k < Nphi
   double2 *ztab = nullptr;                      // chirp-z form: roots, filters, chirp
