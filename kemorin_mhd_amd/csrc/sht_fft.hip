@@ -32,6 +32,22 @@ __device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb) {
   return (b % 8) * per + b / 8;
 }
 
+// Block of lines and component of a work-group of a (line blocks, components)
+// grid.  Where the components of a line are adjacent (the rtp layout) all of
+// them run side by side on one XCD, so that its L2 joins their pieces of a
+// row; component by component each would move whole lines of them: L = 127,
+// Nr = 65, 7 components, forward 318 us, now 175, backward 235, now 186.
+struct FftBlock {
+  long long lines;
+  int nd;
+};
+__device__ __forceinline__ FftBlock fft_block(const FourierAddr &xa) {
+  if (xa.s_line == 1) return FftBlock{(long long)xcd_block(blockIdx.x, gridDim.x), (int)blockIdx.y};
+  const long long id = xcd_group_order((long long)blockIdx.y * gridDim.x + blockIdx.x,
+                                       (long long)gridDim.x * gridDim.y, gridDim.y);
+  return FftBlock{id / gridDim.y, (int)(id % gridDim.y)};
+}
+
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
@@ -285,8 +301,9 @@ __global__ void __launch_bounds__(kFftThreads) k_fft_bwd(
     double *__restrict__ v, const double2 *__restrict__ tw) {
   extern __shared__ double2 buf[];
   const int n = fp.n, B = fp.lines_per_wg, F = B / 2;
-  const int nd = blockIdx.y;
-  const long long line0 = (long long)xcd_block(blockIdx.x, gridDim.x) * B;
+  const FftBlock fb = fft_block(xa);
+  const int nd = fb.nd;
+  const long long line0 = fb.lines * B;
   const long long nnod = nline * n;
   // zero the orders above L
   for (int idx = threadIdx.x; idx < F * (n - 2 * L - 1); idx += kFftThreads) {
@@ -346,8 +363,9 @@ __global__ void __launch_bounds__(kFftThreads) k_fft_fwd(
     FourierAddr xa, const double2 *__restrict__ tw) {
   extern __shared__ double2 buf[];
   const int n = fp.n, B = fp.lines_per_wg, F = B / 2;
-  const int nd = blockIdx.y;
-  const long long line0 = (long long)xcd_block(blockIdx.x, gridDim.x) * B;
+  const FftBlock fb = fft_block(xa);
+  const int nd = fb.nd;
+  const long long line0 = fb.lines * B;
   const long long nnod = nline * n;
   for (int idx = threadIdx.x; idx < F * n; idx += kFftThreads) {
     const int j = idx / F, f = idx - j * F;
@@ -635,8 +653,9 @@ __global__ void __launch_bounds__(NC * NP / 8, 2) k_fft3_bwd(int N, int R0, unsi
   extern __shared__ double2 lds[];
   constexpr int T = NP / 8, NT = NC * T, W = 2 * NC, SS = W + 1;
   const int tid = threadIdx.x, cl = tid / T, j = tid % T;
-  const int nd = blockIdx.y;
-  const long long line0 = (long long)xcd_block(blockIdx.x, gridDim.x) * W;
+  const FftBlock fb = fft_block(xa);
+  const int nd = fb.nd;
+  const long long line0 = fb.lines * W;
   double *stage = reinterpret_cast<double *>(lds);
   constexpr bool TL = fft_bwd_2l<NP>();
   constexpr int NTW = fft_bwd_tw_entries<NP>();
@@ -829,8 +848,9 @@ __global__ void __launch_bounds__(NC * NP / 8, NC * NP / 8 <= 256 ? 2 : 1)
   extern __shared__ double2 lds[];
   constexpr int T = NP / 8, NT = NC * T, W = 2 * NC, SS = W + 1;
   const int tid = threadIdx.x, cl = tid / T, j = tid % T;
-  const int nd = blockIdx.y;
-  const long long line0 = (long long)xcd_block(blockIdx.x, gridDim.x) * W;
+  const FftBlock fb = fft_block(xa);
+  const int nd = fb.nd;
+  const long long line0 = fb.lines * W;
   const long long nnod = nline * N;
   const bool vec2 = (nline & 1) == 0;
   double2 zlo[8], zhi[8];
