@@ -804,6 +804,66 @@ __device__ __forceinline__ int stage_pos(int ctl, int row, int col) {
   return (ctl * 4 * NT + row) * 16 + (KFAST ? col : col ^ (row & 15));
 }
 
+// fwd_vec_store by way of LDS, 16 x 96 doubles of the wave's own: the (r, t, p)
+// of a radius's 32 degrees lie side by side there, so that a store covers runs
+// of three doubles of 21 degrees, some 24 pieces of 64 bytes, instead of 64
+// single doubles apart.  L = 255, Nr = 129, 9 components 1586 -> 1529 us,
+// L = 511, Nr = 257 18.0 -> 17.6 ms.
+__device__ __forceinline__ void fwd_vec_store_lds(const LegDims &d, const d4 (&acc)[2][2][5],
+                                                  int M, int i0, int ct, int lane,
+                                                  double *__restrict__ sp, const SpecAddr &sa,
+                                                  const int *__restrict__ jst,
+                                                  const double *__restrict__ radius,
+                                                  double *__restrict__ lds) {
+  const int L = d.L, nsig = (M == 0) ? 1 : 2;
+  const int ii = i0 + (lane & 15);
+  // element 64 s + lane of two radii: radius, degree and component
+  int kk[3];
+  long long off[3];
+  bool in[3];
+#pragma unroll
+  for (int s = 0; s < 3; s++) {
+    const int e = 64 * s + lane, x = e % 96 / 3;
+    kk[s] = e / 96;
+    off[s] = x * sa.s_j + e % 3 * sa.s_nd;
+    in[s] = M + 2 * i0 + x <= L;
+  }
+  const FwdCol fc = fwd_col(d, ct, lane & 15, d.nv);
+  const int cq = fc.ok ? fc.q : -1;
+  double r1[4], g7[2];
+#pragma unroll
+  for (int r = 0; r < 4; r++) r1[r] = radius[fwd_col(d, ct, 4 * r + (lane >> 4), d.nv).k];
+#pragma unroll
+  for (int par = 0; par < 2; par++) g7[par] = g7_of(M + 2 * ii + par, M);
+#pragma unroll
+  for (int sg = 0; sg < 2; sg++) {
+    if (sg >= nsig) continue;
+    const double ms = (sg == 0) ? (double)M : -(double)M;
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int par = 0; par < 2; par++) {
+        double *o = lds + (4 * r + (lane >> 4)) * 96 + (2 * (lane & 15) + par) * 3;
+        o[0] = r1[r] * r1[r] * g7[par] * acc[sg][par][0][r];
+        o[1] = r1[r] * g7[par] * (acc[sg][par][1][r] - ms * acc[sg][par][2][r]);
+        o[2] = r1[r] * g7[par] * (-acc[sg][par][3][r] - ms * acc[sg][par][4][r]);
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    double *base = sp + (long long)(jst[sg == 0 ? L + M : L - M] + 2 * i0) * sa.s_j;
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+#pragma unroll
+      for (int s = 0; s < 3; s++) {
+        const int c = 2 * j + kk[s], q = __shfl(cq, c), k = __shfl(fc.k, c);
+        const double z = lds[192 * j + 64 * s + lane];
+        if (in[s] && q >= 0) base[off[s] + 3 * q * sa.s_nd + k * sa.s_k] = z;
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 // VEC: components (r, t, p) of a tile of columns; else two tiles of scalars
 template <bool VEC, bool KFAST, int NT>
 __device__ __forceinline__ void leg_fwd_staged(
@@ -970,7 +1030,7 @@ __device__ __forceinline__ void leg_fwd_staged(
     }
   }
   if constexpr (VEC) {
-    fwd_vec_store(d, acc, M, i0, cg * NC + ctl, lane, sp, sa, jst, radius);
+    fwd_vec_store_lds(d, acc, M, i0, cg * NC + ctl, lane, sp, sa, jst, radius, lds + wave * 1536);
   } else {
     d4 q[2][2][2][2];
 #pragma unroll
@@ -1137,8 +1197,8 @@ int launch_leg_bwd(sht_plan *p, int nv, int ns, const double *sp, SpecAddr sa, d
 // Staged from this many waves of a call on: it reads the rows once for four
 // waves but starts and ends them together.  Direct / staged: L = 127, 7
 // components, Nr = 65 (2900 waves) 137 / 147 us, L = 361, 4, Nr = 63 (11000)
-// 826 / 850, L = 255, 9, Nr = 129 (29000) 1590 / 1560, 18, Nr = 65 (29000)
-// 1750 / 1630.
+// 826 / 850, L = 255, 9, Nr = 129 (29000) 1590 / 1529, 18, Nr = 65 (29000)
+// 1750 / 1594.
 constexpr long long kFwdStaged = 16384;
 
 // work-groups of the staged forward: eight times the most of an XCD's orders
