@@ -16,12 +16,13 @@
 // ahead, and waits for no other wave: an FP64 MFMA holds the matrix unit for
 // 64 cycles, so the 8 KB of a step (16 fragments for 20 products) are
 // 6.4 bytes per cycle and SIMD, which L1 and L2 deliver; two waves per SIMD.
-// The matrix units are busy 78 % of the time where a wave has many steps (low
-// orders, L = 511) and about half of it for few steps or where the forward's
-// rows, not multiples of a line, double its L1 accesses.  L = 511, Nr = 257:
+// Large forward calls share their rows through LDS (k_leg_fwd_lds).  The
+// matrix units are busy 78 % of the time in the backward's low orders, which
+// have many steps, half of it in its high ones and 60 % in the forward; a loop
+// of such products alone reaches 72.6 of their 78.6 TF.  L = 511, Nr = 257:
 // backward (8 components) 26.4 ms staged through LDS in its own layout, now
-// 2.3 to pack and 13.2; forward (9) 36.0, now 19.4.  L = 255, Nr = 129:
-// forward (9) 3.14, now 1.6.
+// 2.3 to pack and 13.2; forward (9) 36.0, now 17.6.  L = 255, Nr = 129:
+// forward (9) 3.14, now 1.53.
 //
 // MFMA: v_mfma_f64_16x16x4f64.  A(16x4): lane holds A[lane%16][lane/16];
 // B(4x16): lane holds B[lane/16][lane%16]; D(16x16): lane holds
