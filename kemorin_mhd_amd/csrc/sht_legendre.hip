@@ -1031,6 +1031,9 @@ __device__ __forceinline__ void leg_fwd_staged(
     }
   }
   if constexpr (VEC) {
+    // a last chunk of fewer steps leaves the loop without its barrier: other
+    // waves may still read the rows that the store overwrites
+    __syncthreads();
     fwd_vec_store_lds(d, acc, M, i0, cg * NC + ctl, lane, sp, sa, jst, radius, lds + wave * 1536);
   } else {
     d4 q[2][2][2][2];

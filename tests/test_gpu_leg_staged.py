@@ -66,3 +66,28 @@ def test_large_calls(torch_cuda, L, nr, nth, nv, ns):
             _close(t, w[:, c0:c1], one.view(-1, c1 - c0))
     finally:
         plan.close()
+
+
+@pytest.mark.parametrize("L,nr,nth", [(127, 190, 194), (100, 300, 166)])
+def test_repeats(torch_cuda, L, nr, nth):
+    """A last chunk of fewer than four K steps (25 and 21 of them: 97 and 83 rows):
+    the waves of a work-group leave the product loop without a barrier and turn
+    their results in the LDS that held the rows; repeated calls agree bit for
+    bit."""
+    t = torch_cuda
+    print(f"[gpu] staged forward repeated L={L} Nr={nr} Ntheta={nth}", flush=True)
+    cfg, nv = ShellConfig(L, nr, nth, 2 * nth), 8
+    g = t.Generator(device="cuda")
+    g.manual_seed(L)
+    grid = t.randn(cfg.n_rtp(3 * nv), dtype=t.float64, device="cuda", generator=g)
+    plan = SphTransPlan(cfg, max_ncomp=3 * nv)
+    out = []
+    try:
+        for _ in range(4):
+            w = t.full((cfg.n_rj(3 * nv),), np.nan, dtype=t.float64, device="cuda")
+            plan.sph_forward_transforms(nv, 0, grid, w)
+            out.append(w)
+        t.cuda.synchronize()
+    finally:
+        plan.close()
+    assert all(t.equal(out[0], w) for w in out[1:])
