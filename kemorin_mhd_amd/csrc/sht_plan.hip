@@ -436,9 +436,6 @@ static void free_plan(sht_plan *p) {
       (void)hipEventDestroy(e.second);
     }
   if (p->own_stream) (void)hipStreamDestroy(p->own_stream);
-  if (p->side) (void)hipStreamDestroy(p->side);
-  if (p->ev_fork) (void)hipEventDestroy(p->ev_fork);
-  if (p->ev_join) (void)hipEventDestroy(p->ev_join);
   delete p;
 }
 
@@ -510,14 +507,6 @@ extern "C" int sht_plan_create(const sht_desc *d, sht_plan **out) {
     return SHT_ERR_HIP;
   }
   p->stream = p->own_stream;
-  // side stream for overlapping launches; without it calls run in order
-  if (hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreateWithFlags(&p->ev_fork, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&p->ev_join, hipEventDisableTiming) != hipSuccess) {
-    if (p->side) (void)hipStreamDestroy(p->side);
-    p->side = nullptr;
-    (void)hipGetLastError();
-  }
   // the fixed workspace of sht_backward_noalloc on this device; a failure
   // here is reported by that entry point, which tries again
   (void)scratch_attach(p->device);

@@ -1804,10 +1804,9 @@ static int bwd_split_S(sht_plan *p, const Workspace &ws, int nv, int ns, const d
     int M0 = 0, nM = 0;
     int rc = split_tile<S>(p, st, ti, false, &tb, &M0, &nM);
     if (rc) return rc;
-    // the groups run in order: beside the vector group (ForkJoin, as the
-    // FP64 kernels do) the scalar group only slowed it by as much as it
-    // saved (15.5 against 15.3 ms at L=511), the split GEMMs keeping the
-    // chip busy to their last work-groups
+    // the groups run in order: on a stream beside the vector group the scalar
+    // group only slowed it by as much as it saved (15.5 against 15.3 ms at
+    // L=511), the split GEMMs keeping the chip busy to their last work-groups
     const hipStream_t sm = p->stream;
     for (int i = 0; i < ng; i++) {
       SplitDims d = split_dims(p, ncomp, p->nth_hp / 64);
