@@ -747,12 +747,15 @@ __global__ void __launch_bounds__(256, 2) k_leg_fwd(
 }
 
 // ---------------------------------------------------------------------------
-// Forward, staged: a work-group's rows in LDS, as weighted symmetric and
-// antisymmetric combinations, once for its four waves instead of once a wave.
-// A wave then reads 4 fragments of P a K step from global memory where the
-// direct form reads 16 (rows that start anywhere in a line cost two L1
-// accesses each), and the combinations' FP64 operations, which take the
-// matrix unit's time, are shared.
+// Forward, staged: a work-group's rows in LDS, as symmetric and antisymmetric
+// combinations, once for its four waves instead of once a wave.  A wave then
+// reads 4 fragments of P a K step from global memory where the direct form
+// reads 16 (rows that start anywhere in a line cost two L1 accesses each), and
+// the combinations' FP64 operations, which take the matrix unit's time, are
+// shared.  Weights and 1/sin go to the P fragments and every accumulator takes
+// its K steps in order, as in the direct form: the two give the same bits, so
+// that the choice between them, made for a launch (one tile of orders with P
+// per call), does not show in the results.
 //
 // NT waves along the pair indices by NC = 4 / NT along the columns, as the
 // tiles of an order divide: groups of four tiles (NT = 4), then a remainder of
@@ -921,9 +924,9 @@ __device__ __forceinline__ void leg_fwd_staged(
   auto stage_store = [&](double *buf, int y) {
     const double z = xeq ? 0.0 : xm[y];
     double *o = buf + 2 * y * kPlane + spos;
-    o[0] = (xn[y] + z) * xw.x;
-    o[kPlane] = xeq ? 0.0 : (xn[y] - z) * xw.x;
-    if (VEC && y == 0 && scol == 0 && sct == 0) buf[kBuf + srow] = xw.y;
+    o[0] = xn[y] + z;
+    o[kPlane] = xeq ? 0.0 : xn[y] - z;
+    if (y == 0 && scol == 0 && sct == 0) *reinterpret_cast<double2 *>(buf + kBuf + 2 * srow) = xw;
   };
   // columns of P: an odd block may end before the even one (read what is
   // there: its products are not stored), and a scalar tile's second half with
@@ -957,14 +960,12 @@ __device__ __forceinline__ void leg_fwd_staged(
     for (int u = 0; u < 2; u++)
 #pragma unroll
       for (int c = 0; c < NA; c++) acc[s][u][c] = d4{0.0, 0.0, 0.0, 0.0};
-  auto mul = [&](const Step &f, const double *buf, int s) {
+  auto mul = [&](Step &f, const double *buf, int s) {
     const double *x = buf + stage_pos<KFAST, NT>(ctl, 4 * s + (lane >> 4), lane & 15);
-    double ps[2];
-    if (VEC) {
-      const double as = buf[kBuf + 4 * s + (lane >> 4)];
-      ps[0] = f.a[0][0] * as;
-      ps[1] = f.a[1][0] * as;
-    }
+    const double2 z = *reinterpret_cast<const double2 *>(buf + kBuf + 2 * (4 * s + (lane >> 4)));
+#pragma unroll
+    for (int r = 0; r < 4; r++) f.a[r >> 1][r & 1] *= z.x;
+    const double ps[2] = {f.a[0][0] * z.y, f.a[1][0] * z.y};
 #pragma unroll
     for (int sg = 0; sg < 2; sg++)
 #pragma unroll
@@ -982,27 +983,26 @@ __device__ __forceinline__ void leg_fwd_staged(
           acc[sg][1][0] = mfma64(v, f.a[1][0], acc[sg][1][0]);
         } else {
           // v_t: dP own slot (1), P / sin conjugate slot (4); v_p: 3 and 2
-          const int o = c == 1 ? 1 : 3, z = c == 1 ? 4 : 2;
+          const int o = c == 1 ? 1 : 3, k = c == 1 ? 4 : 2;
           acc[sg][0][o] = mfma64(v, f.a[0][1], acc[sg][0][o]);
           acc[sg][1][o] = mfma64(u, f.a[1][1], acc[sg][1][o]);
-          acc[1 - sg][0][z] = mfma64(u, ps[0], acc[1 - sg][0][z]);
-          acc[1 - sg][1][z] = mfma64(v, ps[1], acc[1 - sg][1][z]);
+          acc[1 - sg][0][k] = mfma64(u, ps[0], acc[1 - sg][0][k]);
+          acc[1 - sg][1][k] = mfma64(v, ps[1], acc[1 - sg][1][k]);
         }
       }
   };
   const int nstep = (d.nth_h + 3) / 4, last = nstep - 1;
-  constexpr int kPitch = kBuf + 16;  // a buffer and 1/sin of its rows
-  Step f[4];
+  constexpr int kPitch = kBuf + 32;  // a buffer and (weight, 1/sin) of its rows
+  Step f[2];
   pload(0, f[0]);
-  pload(last < 1 ? last : 1, f[1]);
   stage_rows(0);
 #pragma unroll
   for (int y = 0; y < 2 * NX; y++) stage_load(y);
 #pragma unroll
   for (int y = 0; y < 2 * NX; y++) stage_store(lds, y);
   __syncthreads();
-  // P two steps ahead; the pairs of the next chunk a few per step, each
-  // written two steps after its load where the chunk has four
+  // P one step ahead; the pairs of the next chunk a few per step, each
+  // written a step after its load where the chunk has four
   constexpr int kPer = NT == 4 ? (2 * NX + 2) / 3 : 2 * NX;
   int cur = 0;
   for (int q = 0; q < nstep; q += 4) {
@@ -1012,12 +1012,12 @@ __device__ __forceinline__ void leg_fwd_staged(
       if (st >= nstep) break;
       const double *buf = lds + cur;
       double *nxt = lds + (kPitch - cur);
-      pload(st + 2 < nstep ? st + 2 : last, f[(s + 2) & 3]);
+      pload(st + 1 < nstep ? st + 1 : last, f[(s + 1) & 1]);
       if (sc == 0) stage_rows(st + NT < nstep ? st / NT + 1 : 0);
 #pragma unroll
       for (int y = sc * kPer; y < (sc + 1) * kPer && y < 2 * NX; y++) stage_load(y);
       __builtin_amdgcn_sched_barrier(0);
-      mul(f[s], buf, sc);
+      mul(f[s & 1], buf, sc);
       __builtin_amdgcn_sched_barrier(0);
       // pairs loaded a step ago (all of them at the end of a shorter chunk)
 #pragma unroll
@@ -1052,7 +1052,7 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2) k_leg_fwd_lds(
     const int *__restrict__ ipad, const double *__restrict__ Pf,
     const double *__restrict__ dPf, const double *__restrict__ radius,
     const double2 *__restrict__ wt) {
-  __shared__ double lds[2 * (12 * kPlane + 16)];
+  __shared__ __align__(16) double lds[2 * (12 * kPlane + 32)];
   const bool vec = blockIdx.x < d.nbv;
   const FwdGroup g = vec ? fwd_group<32>(d, blockIdx.x, (d.ncv + kFwdWaves - 1) / kFwdWaves)
                          : fwd_group<64>(d, blockIdx.x - d.nbv, ((d.ncs + 1) / 2 + kFwdWaves - 1) / kFwdWaves);
@@ -1198,11 +1198,11 @@ int launch_leg_bwd(sht_plan *p, int nv, int ns, const double *sp, SpecAddr sa, d
   return SHT_OK;
 }
 
-// Staged from this many waves of a call on: it reads the rows once for four
-// waves but starts and ends them together.  Direct / staged: L = 127, 7
-// components, Nr = 65 (2900 waves) 137 / 147 us, L = 361, 4, Nr = 63 (11000)
-// 826 / 850, L = 255, 9, Nr = 129 (29000) 1590 / 1529, 18, Nr = 65 (29000)
-// 1750 / 1594.
+// Staged from this many waves of a launch (with P per call, a tile of orders)
+// on: it reads the rows once for four waves but starts and ends them together.
+// Direct / staged: L = 127, 7 components, Nr = 65 (2900 waves) 137 / 147 us,
+// L = 361, 4, Nr = 63 (11000) 826 / 850, L = 255, 9, Nr = 129 (29000) 1590 /
+// 1529, 18, Nr = 65 (29000) 1750 / 1594.
 constexpr long long kFwdStaged = 16384;
 
 // work-groups of the staged forward: eight times the most of an XCD's orders
