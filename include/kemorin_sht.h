@@ -22,7 +22,9 @@
  * All pointers passed to the transform entry points are DEVICE pointers
  * (hipMalloc'd or torch CUDA tensors) unless the name ends in _host.
  * Calls on one plan are stream-ordered on the plan's stream and not
- * re-entrant; different plans may run concurrently.  A plan's own stream is
+ * re-entrant: whole transforms and Legendre stages work in the plan's own
+ * buffers, so calls of one plan on two streams must not overlap (but see
+ * sht_backward_noalloc).  Different plans may run concurrently.  A plan's own stream is
  * a blocking stream; a caller whose inputs are written by work queued on the
  * legacy default stream (asynchronous copies included) binds the plan to
  * hipStreamLegacy with sht_plan_set_stream, so that both share one queue.
@@ -178,9 +180,12 @@ int sht_forward_host(sht_plan *plan, int nvector, int nscalar,
  * allocate device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  The call allocates nothing; its workspace
  * (the Fourier workspace between the Legendre and FFT kernels and, for
- * split-precision plans, the sliced data operand) is a fixed device array of
- * the library, SHT_NOALLOC_SCRATCH_BYTES on each device, in place of the
- * plan's.  Returns SHT_ERR_ARG when the call needs more than that (8 bytes x
+ * split-precision plans, the sliced data operand; FP64 products pack their
+ * spectra into what is left) is a fixed device array of the library,
+ * SHT_NOALLOC_SCRATCH_BYTES on each device, in place of the plan's, which the
+ * call does not touch (with SHT_FLAG_P_ON_THE_FLY it does generate P into the
+ * plan's tile buffers).  Results are those of sht_backward bit for bit.
+ * Returns SHT_ERR_ARG when the call needs more than that (8 bytes x
  * ncomp x (2L+1) x Nr x Ntheta, plus the data slices in split mode: e.g. up
  * to L = 63, Nr = 65, Ntheta = 96 with 9 components in FP64, L = 31, Nr = 33,
  * Ntheta = 48 in split mode) and SHT_ERR_STATE when the plan's stage timers

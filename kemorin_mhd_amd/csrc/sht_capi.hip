@@ -76,7 +76,7 @@ static int leg_bwd(sht_plan *p, const Workspace &ws, int nv, int ns, const doubl
   StageTimer tm(p, 0);
   if (p->digits)
     return launch_leg_bwd_split(p, ws, nv, ns, sp, sa, out, ga);
-  return launch_leg_bwd(p, nv, ns, sp, sa, out, ga);
+  return launch_leg_bwd(p, ws, nv, ns, sp, sa, out, ga);
 }
 static int leg_fwd(sht_plan *p, const Workspace &ws, int nv, int ns, const double *in,
                    GridAddr ga, double *sp, SpecAddr sa) {
@@ -230,8 +230,11 @@ extern "C" int sht_backward_noalloc(sht_plan *p, int nv, int ns, const double *W
     base = scratch_dev[p->device];
   }
   unsigned char *b = (unsigned char *)base;
-  const Workspace ws{(double *)b, db ? (signed char *)(b + xb) : nullptr,
-                     eb ? (int *)(b + xb + db) : nullptr};
+  // behind the Fourier workspace, the sliced operand or the packed spectra
+  const Workspace ws = p->digits ? Workspace{(double *)b, (signed char *)(b + xb),
+                                             (int *)(b + xb + db), nullptr, 0}
+                                 : Workspace{(double *)b, nullptr, nullptr, (double *)(b + xb),
+                                             (kScratchBytes - xb) / (long long)sizeof(double)};
   rc = backward_ws(p, ws, nv, ns, WS_rj, v_rtp);
   if (rc) return rc;
   return check_finite(p, v_rtp, (long long)ncomp * p->nr * p->nth * p->nphi,

@@ -200,14 +200,17 @@ struct StageTimer {
 
 namespace ksht {
 // Per-call workspace of a whole transform: the field-major Fourier workspace
-// between the Legendre and FFT kernels and, for split-precision plans, the
-// sliced data operand (digits and exponents).  Normally the plan's own
-// buffers (plan_workspace); sht_backward_noalloc carves it from the library's
-// fixed device array instead.
+// between the Legendre and FFT kernels, for sliced products the sliced data
+// operand (digits and exponents), and for FP64 ones the packed spectra of a
+// backward (bp_elems doubles; too few for one order: read unpacked).  Normally
+// the plan's own buffers (plan_workspace); sht_backward_noalloc carves it from
+// the library's fixed device array instead.
 struct Workspace {
   double *X;
   signed char *dig;
   int *dexp;
+  double *Bp;
+  long long bp_elems;
 };
 Workspace plan_workspace(const sht_plan *p);
 // bytes of the split engine's data-operand digits and exponents for a call of
@@ -220,8 +223,8 @@ int scratch_attach(int device);
 
 // Legendre launchers (sht_legendre.hip)
 int leg_init(sht_plan *p);
-int launch_leg_bwd(sht_plan *p, int nv, int ns, const double *sp, SpecAddr sa,
-                   double *out, GridAddr ga);
+int launch_leg_bwd(sht_plan *p, const Workspace &ws, int nv, int ns, const double *sp,
+                   SpecAddr sa, double *out, GridAddr ga);
 int launch_leg_fwd(sht_plan *p, int nv, int ns, const double *in, GridAddr ga,
                    double *sp, SpecAddr sa);
 // FFT launchers (sht_fft.hip)

@@ -1151,12 +1151,15 @@ static LegDims make_dims(const sht_plan *p, int nv, int ns) {
 static int group_waves(long long waves) { return waves < 1024 ? 1 : 4; }
 static unsigned groups(long long waves, int nw) { return (unsigned)((waves + nw - 1) / nw); }
 
-int launch_leg_bwd(sht_plan *p, int nv, int ns, const double *sp, SpecAddr sa, double *out,
-                   GridAddr ga) {
+int launch_leg_bwd(sht_plan *p, const Workspace &ws, int nv, int ns, const double *sp,
+                   SpecAddr sa, double *out, GridAddr ga) {
   LegDims d = make_dims(p, nv, ns);
-  const long long W = d.W, cap = p->bp_elems > 0 ? p->bp_elems : 1;
+  const long long W = d.W, cap = ws.bp_elems > 0 ? ws.bp_elems : 1;
   const long long per_v = (long long)d.ncv * d.ntv, per_s = (long long)((d.ncs + 1) / 2) * d.nts;
-  const bool pack = packs(p, nv, ns);
+  // the fixed workspace may not hold one order's rows beside the call's
+  // Fourier workspace: unpacked then, the same products in the same order (its
+  // calls are far below the 32-bit offsets that packs() asks about)
+  const bool pack = packs(p, nv, ns) && cap >= pack_rows(p->L + 1) * W;
   int dt = 1;  // degrees of a packed run
   while (2 * dt * d.ncomp <= kPackRun) dt *= 2;
   for (int ti = 0; ti < ptile_count(p); ti++) {
@@ -1179,7 +1182,7 @@ int launch_leg_bwd(sht_plan *p, int nv, int ns, const double *sp, SpecAddr sa, d
         const int nz = (int)((pack_rows(p->L - M0 + 1) + dt - 1) / dt);
         const long long nb = (p->nr + 15) / 16 * 2LL * d.nM * nz;
         hipLaunchKernelGGL(k_leg_pack, dim3((unsigned)nb), dim3(256), 0, p->stream, d, dt, nz, sp,
-                           sa.s_k, p->t.jst, p->Bp);
+                           sa.s_k, p->t.jst, ws.Bp);
         KSHT_HIP(hipGetLastError());
       }
       StageTimer tk(p, 5);
@@ -1187,7 +1190,7 @@ int launch_leg_bwd(sht_plan *p, int nv, int ns, const double *sp, SpecAddr sa, d
       d.nbv = groups(d.nM * per_v, nw);
       const dim3 g(d.nbv + groups(d.nM * per_s, nw)), bl(64 * nw);
       if (pack)
-        hipLaunchKernelGGL(k_leg_bwd<true>, g, bl, 0, p->stream, d, p->Bp, sa.s_k, out, ga,
+        hipLaunchKernelGGL(k_leg_bwd<true>, g, bl, 0, p->stream, d, ws.Bp, sa.s_k, out, ga,
                            p->t.jst, pt.offb, p->t.ipad, pt.Pb, pt.dPb, p->t.a_r, p->t.asin_t);
       else
         hipLaunchKernelGGL(k_leg_bwd<false>, g, bl, 0, p->stream, d, sp, sa.s_k, out, ga,

@@ -1737,7 +1737,7 @@ void split_ws_bytes(const sht_plan *p, int ncomp, bool backward, long long *dig_
 
 Workspace plan_workspace(const sht_plan *p) {
   const SplitState *st = (const SplitState *)p->split;
-  return Workspace{p->X, st ? st->dig : nullptr, st ? st->dexp : nullptr};
+  return Workspace{p->X, st ? st->dig : nullptr, st ? st->dexp : nullptr, p->Bp, p->bp_elems};
 }
 
 static SplitDims split_dims(const sht_plan *p, int ncomp, int nblk) {
