@@ -139,8 +139,10 @@ int sht_plan_get_variant(const sht_plan *plan, const char *name, int *value);
  * Replaces select_legendre_transform (MS/init_sphrical_transform_MHD.f90:
  * 201-345), which times the reference's Legendre loop variants at start-up.
  * cache_path (NULL = none): a JSON file of earlier results, one entry per
- * shape (L, Nr, Ntheta, Nphi, precision, slices, flags, field sets); a hit
- * sets the cached winner without timing, a miss appends the new winner.
+ * shape (L, Nr, Ntheta, Nphi, precision, slices, sliced or FP64 products,
+ * flags, field sets) and kernel set of the library, so that files of other
+ * versions are timed again; a hit sets the cached winner without timing, a
+ * miss appends the new winner.
  * ms_out (NULL = none): [round-trip ms of the winner, of the default].
  * Allocates temporary device buffers of the field sets' size; runs on the
  * plan's stream and returns after it drained. */

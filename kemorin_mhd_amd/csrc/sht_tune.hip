@@ -18,9 +18,9 @@
 // stream) decides.  Results are cached in a JSON file, one entry per line:
 //   {"key": "<shape>", "split_fwd_mfma": 16, "fft_form": 1, "ms": 51.2,
 //    "default_ms": 52.9}
-// keyed by L, Nr, Ntheta, Nphi, precision, slices, tables per call and the
-// field sets, so a later plan of the same shape reads its winner instead of
-// timing.  The outputs do not depend on the variant (each variant is held to
+// keyed by the kernel set, L, Nr, Ntheta, Nphi, precision, slices, whether the
+// products run sliced, tables per call and the field sets, so a later plan of
+// the same shape reads its winner instead of timing.  The outputs do not depend on the variant (each variant is held to
 // the same parity bars), only the time.
 #include <cmath>
 #include <cstdio>
@@ -38,11 +38,18 @@ __global__ void k_tune_fill(double *x, long long n, double scale) {
   if (i < n) x[i] = scale * sin(0.7 * (double)(i % 100003) + 0.3);
 }
 
+// What a variant's value stands for, as a number: raised when a form's kernels
+// or meaning change, so that entries timed on other kernels are timed again
+// (0: files without it; 1: fft_form 1 includes the folded DFT, FP64 products
+// below a truncation).
+constexpr int kKernelSet = 1;
+
 static std::string tune_key(const sht_plan *p, int nvb, int nsb, int nvf, int nsf) {
   char buf[256];
-  snprintf(buf, sizeof buf, "L=%d nr=%d nth=%d nphi=%d prec=%d slices=%d p_otf=%d bwd=%d,%d fwd=%d,%d",
-           p->L, p->nr, p->nth, p->nphi, p->precision, p->n_slices, p->p_otf, nvb, nsb, nvf,
-           nsf);
+  snprintf(buf, sizeof buf,
+           "kernels=%d L=%d nr=%d nth=%d nphi=%d prec=%d slices=%d sliced=%d p_otf=%d bwd=%d,%d fwd=%d,%d",
+           kKernelSet, p->L, p->nr, p->nth, p->nphi, p->precision, p->n_slices, p->digits ? 1 : 0,
+           p->p_otf, nvb, nsb, nvf, nsf);
   return buf;
 }
 
