@@ -115,18 +115,19 @@ long long sht_plan_device_bytes(const sht_plan *plan);
  *                     faster (precision, above), or sliced ones at every size
  *                     (their tables are set up, and counted in the plan's
  *                     device bytes, when first selected);
- *   "fft_form":       1, 0, 2 or 3: the default by length (the split-form
+ *   "fft_form":       1, 0, 2, 3 or 4: the default by length (the split-form
  *                     FFT where Nphi = r0 2^k, 2^k > L, and Nphi >= 384; the
  *                     mixed-radix FFT where its radices are 2 and 3, or up
  *                     to 13, and L is large; a folded real DFT on FP64 MFMA
  *                     otherwise), the mixed-radix Stockham FFT, the pruned
- *                     real DFT as one
- *                     FP64 GEMM per direction against a cos/sin basis, or
- *                     the whole line as one chirp-z (Bluestein) convolution
- *                     of power-of-two length MP >= Nphi + 2L (MP <= 2048; any
- *                     prime factors).  Forms 2 and 3 set up their tables (and
- *                     count them in the plan's device bytes) when first
- *                     selected; SHT_ERR_UNSUPPORTED where they do not apply.
+ *                     real DFT as one FP64 GEMM per direction against a
+ *                     cos/sin basis, the whole line as one chirp-z
+ *                     (Bluestein) convolution of power-of-two length
+ *                     MP >= Nphi + 2L (MP <= 2048; any prime factors), or the
+ *                     split-form FFT also below 384.  Forms 2 and 3 set up
+ *                     their tables (and count them in the plan's device bytes)
+ *                     when first selected; SHT_ERR_UNSUPPORTED where a form
+ *                     does not apply.
  * Results do not depend on the variant beyond round-off.  SHT_ERR_ARG for an
  * unknown name or value. */
 int sht_plan_set_variant(sht_plan *plan, const char *name, int value);

@@ -163,8 +163,9 @@ struct sht_plan {
   // SHT_FLAG_CHECK_FINITE: device counter of non-finite outputs (else null)
   unsigned long long *nonfinite = nullptr;
   // FFT form: 1 = by length (zfold_wins: split form n = r0 * 2^k, folded DFT
-  // or mixed radix), 0 = the mixed-radix Stockham form for every length, 2 = the pruned real DFT as an
-  // FP64 GEMM (set-up on first selection: sht_dft.hip)
+  // or mixed radix), 0 = the mixed-radix Stockham form for every length, 2 = the
+  // pruned real DFT as an FP64 GEMM (set-up on first selection: sht_dft.hip),
+  // 3 = chirp-z (likewise), 4 = the split form where the length has it
   int var_fft_form = 1;
   void *dft = nullptr;
   // stage timers (sht_plan_timer_*): event pairs recorded per launch

@@ -601,7 +601,7 @@ extern "C" long long sht_plan_device_bytes(const sht_plan *p) { return p ? p->de
 
 // Kernel variants: name -> the plan field and its allowed values.
 static int *variant_slot(sht_plan *p, const char *name, const int **allowed, int *nallowed) {
-  static const int mfma[] = {16, 32}, form[] = {0, 1, 2, 3}, onoff[] = {0, 1};
+  static const int mfma[] = {16, 32}, form[] = {0, 1, 2, 3, 4}, onoff[] = {0, 1};
   if (!strcmp(name, "split_fwd_mfma")) {
     *allowed = mfma;
     *nallowed = 2;
@@ -619,7 +619,7 @@ static int *variant_slot(sht_plan *p, const char *name, const int **allowed, int
   }
   if (!strcmp(name, "fft_form")) {
     *allowed = form;
-    *nallowed = 4;
+    *nallowed = 5;
     return &p->var_fft_form;
   }
   return nullptr;
@@ -643,6 +643,10 @@ extern "C" int sht_plan_set_variant(sht_plan *p, const char *name, int value) {
       if (slot == &p->var_fft_form && (value == 2 || value == 3)) {
         const int rc = value == 2 ? dft_init(p) : czt_init(p);
         if (rc) return rc;
+      }
+      if (slot == &p->var_fft_form && value == 4 && !p->fft.fast) {
+        set_error("sht_plan_set_variant: no split-form FFT for L = %d, Nphi = %d", p->L, p->nphi);
+        return SHT_ERR_UNSUPPORTED;
       }
       if (slot == &p->var_split_all && value == 1 && p->precision == SHT_PREC_SPLIT_INT8 &&
           !p->split) {

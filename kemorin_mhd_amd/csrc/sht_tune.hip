@@ -7,11 +7,11 @@
 // fastest for the run.  Here the variants are the kernel forms of one plan:
 //   split_fwd_mfma  16 or 32: INT8 MFMA form of the forward split products
 //                   (split-precision plans);
-//   fft_form        1, 0, 2 or 3: the default by length (split-form FFT,
-//                   folded DFT or mixed radix), mixed-radix Stockham FFT, the
-//                   pruned real DFT as an FP64 GEMM (sht_dft.hip), or the
-//                   whole line as
-//                   one chirp-z (Bluestein) convolution of power-of-two
+//   fft_form        1, 0, 4, 2 or 3: the default by length (split-form FFT,
+//                   folded DFT or mixed radix), mixed-radix Stockham FFT,
+//                   split-form FFT where the default is another, the pruned
+//                   real DFT as an FP64 GEMM (sht_dft.hip), or the whole line
+//                   as one chirp-z (Bluestein) convolution of power-of-two
 //                   length (sht_fft.hip).
 // Every combination runs one backward and one forward transform untimed,
 // then the best of three timed round trips (HIP events on the plan's
@@ -150,6 +150,7 @@ extern "C" int sht_plan_autotune(sht_plan *p, int nvb, int nsb, int nvf, int nsf
   std::vector<int> mfmas = {16}, forms = {1};
   if (p->digits) mfmas.push_back(32);
   if (p->fft.fast || p->t.zfb) forms.push_back(0);  // else form 1 is form 0
+  if (p->fft.fast && p->t.zfb) forms.push_back(4);  // else form 1 is form 4, if any
   if (dft_init(p) == SHT_OK) forms.push_back(2);  // the DFT product, where its set-up fits
   if (czt_init(p) == SHT_OK) forms.push_back(3);  // the chirp-z form, Nphi + 2L <= 2048
   const int keep_mfma = p->var_fwd_mfma, keep_form = p->var_fft_form;
