@@ -114,10 +114,15 @@ __global__ void __launch_bounds__(256, 2) k_zfold_bwd(ZfoldDims d, const double 
     for (int rt = 0; rt < 2; rt++)
 #pragma unroll
       for (int ct = 0; ct < 2; ct++) acc[ty][rt][ct] = d4{0.0, 0.0, 0.0, 0.0};
-  // rows past the last order repeat it (their table entries are zero), and
-  // the sine row of m = 0 is the cosine's (sin 0 = 0)
-  auto load = [&](int ks, d2 (&a)[4], d2 (&b)[4]) {
-    const int i = ks * 4 + kq;
+  // The highest orders first: coefficients fall with m, so the partial sums
+  // stay small until the last steps.  Falling as (m + 1)^-1.5, N = 192, 540,
+  // 1086, relative L2 against 80-bit sums: 1.2e-16 each; lowest first 2.6, 4.5,
+  // 6.3e-16, the mixed-radix FFT 1.3, 1.8, 2.4e-16.  Equal coefficients, either
+  // order: 2.1, 3.3, 4.6e-16, the FFT 1.8, 2.6, 2.9e-16.
+  // Rows past the last order repeat it (their table entries are zero), and
+  // the sine row of m = 0 is the cosine's (sin 0 = 0).
+  auto load = [&](int step, d2 (&a)[4], d2 (&b)[4]) {
+    const int ks = d.k4 - 1 - step, i = ks * 4 + kq;
     const int me = 2 * i < Le ? 2 * i : Le, mo = 2 * i + 1 < Lo ? 2 * i + 1 : Lo;
     const int f = xa.fftpack;
     const int qe = me ? 2 * me - 1 + f : 0, qs = me ? qe + 1 : 0, qo = 2 * mo - 1 + f;
@@ -184,6 +189,10 @@ __global__ void __launch_bounds__(256, 2) k_zfold_fwd(ZfoldDims d, const double 
 #pragma unroll
       for (int ct = 0; ct < 2; ct++) acc[ty][rt][ct] = d4{0.0, 0.0, 0.0, 0.0};
   const unsigned ls = (unsigned)d.nline;
+  // No such order here: the points weigh alike, and a sum of N/4 rounds more
+  // than an FFT's log N levels: N = 192, 540, 1086, 2160 2.7, 4.4, 6.6, 8.7e-16
+  // against 1.6, 2.0, 3.0, 2.2e-16.  The Legendre sums of a whole transform add
+  // ten times that and more, and its error is the same with either.
   // j = 0 reads x_0 and x_H twice and j = N/4 its two points twice: their
   // table entries are halved; rows past N/4 repeat it against zeros
   auto load = [&](int ks, d2 (&a)[4], d2 (&b)[4]) {
