@@ -303,10 +303,10 @@ def run_engine(cfg, precision, args, torch, sp_b, grid_f, keep=False, otf=False,
     timers = plan.timer_read()
     plan.timer_enable(False)
     dev_bytes = plan.device_bytes()
-    # the split backward's vector launches also take one scalar each (5 or 6
+    # the sliced backward's vector launches also take one scalar each (5 or 6
     # slices, the default variant): 2 x (5 + 1) contractions in one kernel
-    fused = (precision == "split" and (args.slices or 6) <= 6
-             and plan.get_variant("split_bwd_fused") == 1)
+    sliced, fft = bool(plan.get_variant("sliced")), plan.get_variant("fft_kernels")
+    fused = sliced and (args.slices or 6) <= 6 and plan.get_variant("split_bwd_fused") == 1
     plan.close()
     out = (grid_b, sp_f) if keep else None
     if not keep:
@@ -316,7 +316,7 @@ def run_engine(cfg, precision, args, torch, sp_b, grid_f, keep=False, otf=False,
     return dict(ms_per_step=ms, round_trips_per_s=1e3 / ms, timers=timers, plan_bytes=dev_bytes,
                 outputs=out, slices=(args.slices or 6) if precision == "split" else 0,
                 hbm_in_use_bytes=total_b - free_b, hbm_total_bytes=total_b, autotune=tuned,
-                bwd_fused=fused, steps=args.steps)
+                bwd_fused=fused, steps=args.steps, otf=otf, sliced=sliced, fft=fft)
 
 
 FIELDS_BWD = (("vector1", 0, 3), ("vector2", 3, 6), ("scalar1", 6, 7), ("scalar2", 7, 8))
@@ -383,40 +383,55 @@ def hbm_traffic(engine, kernel):
     return None
 
 
+def kernel_names(cfg_d, res, slices):
+    """The kernels that the round trip's stages run on: the plan says whether
+    its products are sliced and which zonal form it takes; the FP64 Legendre
+    kernels go by the waves of a launch (sht_legendre.hip: packed spectra from
+    2048, rows staged in LDS from 16384)."""
+    L, nr, rows = cfg_d["L"], cfg_d["nr"], (cfg_d["nth"] + 1) // 2
+    up = lambda a, b: -(-a // b)
+    if res["sliced"]:
+        bwd = f"ksht::k_leg_bwd_split<{slices}, {4 if res['bwd_fused'] else 3}, true>"
+        fwd = f"ksht::k_leg_fwd_split<{slices}, 3, true>"
+    else:
+        wb = (L + 1) * (up(2 * nr, 16) * up(rows, 16) + up(up(2 * nr, 16), 2) * up(rows, 32))
+        wf = sum(up(n, 32) for n in range(1, L + 2)) * up(3 * nr, 16)
+        if res["otf"]:
+            wf //= 8  # a launch is a tile of orders, about an eighth
+        bwd = f"ksht::k_leg_bwd<{'true' if wb >= 2048 else 'false'}>"
+        fwd = "ksht::k_leg_fwd_lds<true>" if wf >= 16384 else "ksht::k_leg_fwd"
+    npow = 32  # split form: the smallest power of two above L
+    while npow < L + 1:
+        npow *= 2
+    zb, zf = {0: ("ksht::k_fft_bwd (mixed radix)", "ksht::k_fft_fwd (mixed radix)"),
+              2: ("DFT product (library GEMM)", "DFT product (library GEMM)"),
+              3: ("ksht::k_fftz_bwd", "ksht::k_fftz_fwd"),
+              4: (f"ksht::k_fft3_bwd<{npow}, {2 if npow >= 1024 else 4}>",
+                  f"ksht::k_fft3_fwd<{npow}, {8 if npow <= 512 else 4}>"),
+              5: ("ksht::k_zfold_bwd<true>", "ksht::k_zfold_fwd<true>")}[res["fft"]]
+    return {"legendre_backward_vector_kernel": bwd, "legendre_forward_vector_kernel": fwd,
+            "fft_backward": zb, "fft_forward": zf}
+
+
 def kernel_roofline(cfg_d, res, precision, slices):
     """Roofline of the round trip's dominant kernel.  Legendre kernels: the
-    vector-group kernel alone (stage timers 5/6, HIP events on the plan's
-    stream), algorithmic work = FP64 flops of its contractions (10 F1 backward:
-    2 vectors x 5, or 12 F1 where the split backward's vector launch also
-    takes the two scalars; 15 F1 forward: 3 vectors x 5); in the split engine each FP64
-    multiply-add is S(S+1)/2 INT8 slice products, so its INT8 work is that
+    product kernel alone (stage timers 5/6, HIP events on the plan's stream),
+    algorithmic work = FP64 flops of its contractions (backward 12 F1: 2 vectors
+    x 5 and two scalars, or 10 F1 where the sliced scalars have launches of
+    their own; forward 15 F1: 3 vectors x 5); in sliced products each FP64
+    multiply-add is S(S+1)/2 INT8 slice products, so their INT8 work is that
     many times the FP64 flops, against the INT8 MFMA peak.  FFT stages: the
     bytes a launch must move (X in, grid out, or the reverse)."""
     F1 = flops_per_contraction(cfg_d)
     nline = cfg_d["nr"] * cfg_d["nth"]
     nslot = 2 * cfg_d["L"] + 1
     tri = slices * (slices + 1) // 2
-    # the plan's FFT form: split form Nphi = R0 NP (NP the smallest power of two
-    # above L, 32..512) with 4 (backward) and 8 (forward) complex lines per
-    # work-group, else the mixed-radix kernels
-    npow = 32
-    while npow < cfg_d["L"] + 1:
-        npow *= 2
-    fast = npow <= 512 and cfg_d["nphi"] % npow == 0
-    split = precision == "split"
-    kname = {
-        "legendre_backward_vector_kernel": (
-            f"ksht::k_leg_bwd_split<{slices}, {4 if res.get('bwd_fused') else 3}, true>" if split
-            else "ksht::k_leg_bwd<true>"),
-        "legendre_forward_vector_kernel": (f"ksht::k_leg_fwd_split<{slices}, 3, true>" if split
-                                           else "ksht::k_leg_fwd"),
-        "fft_backward": f"ksht::k_fft3_bwd<{npow}, 4>" if fast else "ksht::k_fft_bwd (mixed radix)",
-        "fft_forward": f"ksht::k_fft3_fwd<{npow}, 8>" if fast else "ksht::k_fft_fwd (mixed radix)",
-    }
+    split = res["sliced"]
+    kname = kernel_names(cfg_d, res, slices)
     stages = {
         # the FP64 kernel takes vectors and scalars in one launch
         "legendre_backward_vector_kernel": (
-            "mfma", (12 if res.get("bwd_fused") or not split else 10) * F1),
+            "mfma", (12 if res["bwd_fused"] or not split else 10) * F1),
         "legendre_forward_vector_kernel": ("mfma", 15 * F1),
         "fft_backward": ("hbm", 8.0 * 8 * nline * (nslot + cfg_d["nphi"])),
         "fft_forward": ("hbm", 8.0 * 9 * nline * (nslot + cfg_d["nphi"])),
@@ -592,7 +607,7 @@ def main():
         "value": res["round_trips_per_s"], "unit": "round_trips/s",
         "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": res["ms_per_step"], "higher_is_better": True, "scaling": "weak",
-        "vs_baseline": None, "dtype": "f64" if head == "fp64" else "f64 (int8-sliced Legendre)",
+        "vs_baseline": None, "dtype": "f64 (int8-sliced Legendre)" if res["sliced"] else "f64",
         "data": "synthetic (seeded Gaussian spectra, sigma=(l+1)^-1.5 sin(pi(r-ri)/(ro-ri)))",
         "config": {"workload": (f"round trip L={cfg_d['L']} Nr={cfg_d['nr']} "
                                 f"Ntheta={cfg_d['nth']} Nphi={cfg_d['nphi']}: backward 2 vector + "

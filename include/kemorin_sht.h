@@ -128,6 +128,10 @@ long long sht_plan_device_bytes(const sht_plan *plan);
  *                     their tables (and count them in the plan's device bytes)
  *                     when first selected; SHT_ERR_UNSUPPORTED where a form
  *                     does not apply.
+ * Read only, what these and the sizes come to: "sliced", 1 where the plan's
+ * Legendre products run on INT8 slices; "fft_kernels", what a whole transform's
+ * zonal stage runs on: 0 mixed radix, 2 DFT product, 3 chirp-z, 4 split form,
+ * 5 folded DFT.
  * Results do not depend on the variant beyond round-off.  SHT_ERR_ARG for an
  * unknown name or value. */
 int sht_plan_set_variant(sht_plan *plan, const char *name, int value);

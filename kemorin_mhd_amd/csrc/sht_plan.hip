@@ -677,6 +677,19 @@ extern "C" int sht_plan_get_variant(const sht_plan *p, const char *name, int *va
     set_error("sht_plan_get_variant: null argument");
     return SHT_ERR_ARG;
   }
+  // what the variants and the rules of sizes come to, read only
+  if (!strcmp(name, "sliced")) {
+    *value = p->digits ? 1 : 0;
+    return SHT_OK;
+  }
+  if (!strcmp(name, "fft_kernels")) {
+    const int f = p->var_fft_form;
+    *value = (f == 2 && p->dft) || (f == 3 && p->fft.zm) ? f
+             : f == 1 && p->t.zfb                        ? 5
+             : f && p->fft.fast                          ? 4
+                                                         : 0;
+    return SHT_OK;
+  }
   const int *allowed = nullptr;
   int n = 0;
   int *slot = variant_slot(const_cast<sht_plan *>(p), name, &allowed, &n);
