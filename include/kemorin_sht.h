@@ -58,8 +58,8 @@ typedef struct {
   const double *radius; /* host array of Nr radii                        */
   int max_ncomp;    /* largest ncomp a call will pass (workspace size)    */
   int precision;    /* SHT_PREC_FP64 or SHT_PREC_SPLIT_INT8: products of  */
-                    /* INT8 slices where they are the faster ones (L from */
-                    /* 448 on; 5 slices 384, 4 slices 224), FP64 below    */
+                    /* INT8 slices from L = 448 on (5 slices 384, 4 slices */
+                    /* 224), FP64 below, where those are faster           */
   int n_slices;     /* split mode: INT8 slices per operand (0 = default) */
   int flags;        /* SHT_FLAG_* bits, 0 for none                      */
 } sht_desc;
@@ -86,7 +86,10 @@ typedef struct {
  * Legendre/FFT set-up it runs: Gauss points with the reference's Newton
  * loop (MHD/Fortran_src/CORE_src/gauss_integration/gauss_integration.f90:60),
  * Schmidt P_l^m and dP/dtheta generated on the GPU in FP64, 1/sin(theta),
- * index stacks and FFT twiddles.  The plan owns all device memory. */
+ * index stacks and FFT twiddles.  The plan owns all device memory.  A plan
+ * that runs FP64 products on more than a small shell keeps, beside tables and
+ * Fourier workspace, the packed spectra of a backward: of all orders up to
+ * 1 GiB, fewer at a time above that or where memory is short. */
 int sht_plan_create(const sht_desc *desc, sht_plan **plan);
 int sht_plan_destroy(sht_plan *plan);
 /* Run subsequent work on this hipStream_t (NULL = plan's own stream;
@@ -111,8 +114,8 @@ long long sht_plan_device_bytes(const sht_plan *plan);
  *                     5 or 6 slices), or the scalars run in launches of
  *                     their own (0); the results are the same bit for bit;
  *   "split_all":       0 (default) or 1: a split-precision plan runs FP64
- *                     products below the truncations where sliced ones are
- *                     faster (precision, above), or sliced ones at every size
+ *                     products below the truncations where they are the
+ *                     faster ones (precision, above), or sliced at every size
  *                     (their tables are set up, and counted in the plan's
  *                     device bytes, when first selected);
  *   "fft_form":       1, 0, 2, 3 or 4: the default by length (the split-form
@@ -159,9 +162,11 @@ int sht_plan_autotune(sht_plan *plan, int nvector_b, int nscalar_b, int nvector_
  * 22 Legendre backward, 23 Legendre forward, 24 FFT, 18-21 exchanges).
  * When enabled, every kernel launch of the plan is bracketed by HIP events
  * on the plan's stream.  Stage ids: 0 Legendre backward, 1 FFT backward,
- * 2 FFT forward, 3 Legendre forward, 4 exchanges; 5 and 6 time the
- * vector-group Legendre kernel alone (backward, forward; inside 0 and 3,
- * without the operand slicing of the split engine).
+ * 2 FFT forward, 3 Legendre forward, 4 exchanges; 5 and 6 time the kernels
+ * of the Legendre products alone (backward, forward; inside 0 and 3): those
+ * of all fields in FP64, without the packing of the spectra, and those of the
+ * vector groups in sliced products, without the slicing.  A call counts one
+ * launch per tile of orders (P per call) and per share of packed spectra.
  * sht_plan_timer_read synchronises, returns per-stage total milliseconds and
  * launch counts (n entries each, n <= 7) and resets the counters. */
 int sht_plan_timer_enable(sht_plan *plan, int on);

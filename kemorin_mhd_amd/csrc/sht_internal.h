@@ -18,8 +18,8 @@ typedef int i4 __attribute__((ext_vector_type(4)));
 
 constexpr int kTile = 16;   // MFMA tile edge (rows, radii, degrees)
 constexpr int kMaxPass = 24;
-// Legendre bwd, FFT bwd, FFT fwd, Legendre fwd, exchanges, and the vector-group
-// Legendre kernels alone (bwd, fwd): the dominant kernels of a round trip
+// Legendre bwd, FFT bwd, FFT fwd, Legendre fwd, exchanges, and the kernels of
+// the Legendre products alone (bwd, fwd): the dominant ones of a round trip
 constexpr int kNumStages = 7;
 
 void set_error(const char *fmt, ...);
@@ -266,16 +266,19 @@ int pole_tables_init(sht_plan *p);
 // split precision (sht_split.hip)
 int split_init(sht_plan *p);
 void split_free(sht_plan *p);
-// Whether the sliced products of a split-precision plan beat its FP64 ones,
-// which need no slicing pass over the data.  Legendre stages, backward /
+// Whether a split-precision plan runs sliced products: below these truncations
+// its FP64 ones, which need no slicing pass over the data, are the faster ones
+// by far; above, the two are level at first and sliced ones ahead at the
+// largest, so a plan runs what it was asked for.  Legendre stages, backward /
 // forward, sliced against FP64: 6 slices L = 127, Nr = 65, 8 and 7 components
 // 286 / 271 against 153 / 178 us, L = 255, 9 components 1098 / 1000 against
 // 822 / 795, L = 361, 4, Nr = 63 925 / 1071 against 824 / 826, L = 511, 8, Nr
-// = 65 4.07 / 4.66 against 4.04 / 4.46 ms, 9, Nr = 257 18.0 / 18.1 against
-// 17.8 / 18.2, L = 1023, 8 34.2 / 46.8 against 35.0 / 44.2.  5 slices, 9
-// components, Nr = 65: L = 255 957 / 885 us, L = 511 4.49 / 4.45 against 4.61
-// / 4.94 ms.  4 slices: L = 191 559 / 514 against 421 / 421 us, L = 255 814 /
-// 773.
+// = 65 4.07 / 4.66 against 4.04 / 4.46 ms, 8 and 9, Nr = 257 13.8 / 18.0
+// against 14.6 / 17.0, L = 1023, 8, Nr = 65 34.2 / 46.8 against 35.0 / 44.2, 8
+// and 9, Nr = 257 with P per call 87 / 116 against 96 / 131.  5 slices, 9
+// components, Nr = 65: L = 255 957 / 885 us against 822 / 795, L = 511 4.49 /
+// 4.45 against 4.61 / 4.94 ms.  4 slices: L = 191 559 / 514 against 421 / 421
+// us, L = 255 814 / 773 against 822 / 795.
 inline bool split_wins(int L, int n_slices) {
   return L >= (n_slices >= 6 ? 448 : n_slices == 5 ? 384 : 224);
 }

@@ -18,11 +18,11 @@
 // 6.4 bytes per cycle and SIMD, which L1 and L2 deliver; two waves per SIMD.
 // Large forward calls share their rows through LDS (k_leg_fwd_lds).  The
 // matrix units are busy 78 % of the time in the backward's low orders, which
-// have many steps, half of it in its high ones and 60 % in the forward; a loop
-// of such products alone reaches 72.6 of their 78.6 TF.  L = 511, Nr = 257:
-// backward (8 components) 26.4 ms staged through LDS in its own layout, now
-// 2.3 to pack and 13.2; forward (9) 36.0, now 17.6.  L = 255, Nr = 129:
-// forward (9) 3.14, now 1.53.
+// have many steps, half of it in its high ones (68 % of a call at L = 511) and
+// 67 % in the forward; a loop of such products alone reaches 72.6 of their 78.6
+// TF.  L = 511, Nr = 257: backward (8 components) 26.4 ms staged through LDS in
+// its own layout, now 2.1 to pack and 12.5 to 13.2; forward (9) 36.0, now 17.1.
+// L = 255, Nr = 129: forward (9) 3.14, now 1.45.
 //
 // MFMA: v_mfma_f64_16x16x4f64.  A(16x4): lane holds A[lane%16][lane/16];
 // B(4x16): lane holds B[lane/16][lane%16]; D(16x16): lane holds
@@ -1203,9 +1203,10 @@ int launch_leg_bwd(sht_plan *p, const Workspace &ws, int nv, int ns, const doubl
 
 // Staged from this many waves of a launch (with P per call, a tile of orders)
 // on: it reads the rows once for four waves but starts and ends them together.
-// Direct / staged: L = 127, 7 components, Nr = 65 (2900 waves) 137 / 147 us,
-// L = 361, 4, Nr = 63 (11000) 826 / 850, L = 255, 9, Nr = 129 (29000) 1590 /
-// 1529, 18, Nr = 65 (29000) 1750 / 1594.
+// Direct / staged: L = 127, 7 components, Nr = 65 (2900 waves) 143 / 163 us,
+// L = 361, 4, Nr = 63 (11000) 834 / 820, L = 255, 9, Nr = 129 (29000) 1593 /
+// 1446, 18, Nr = 65 (29000) 1756 / 1515, L = 511, 9, Nr = 257 (210000) 17.2 ms
+// both.
 constexpr long long kFwdStaged = 16384;
 
 // work-groups of the staged forward: eight times the most of an XCD's orders
